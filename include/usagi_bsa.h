@@ -26,12 +26,15 @@
  *     and its return value), or NULL / 0 for the kernel's built-in order. Any plan of the same
  *     CSR gives bit-identical results: it only decides which GPU slot runs which query block.
  *   - stream: a hipStream_t (NULL = the default stream). The launch is asynchronous.
- *   - Kernel: calls without seq_lens whose rows hold at most 4 key blocks on average
- *     (max_nnz <= 4 * T/128, or the analytic pattern's own count) run a software-pipelined
- *     kernel; other calls, and every call when USAGI_BSA_PIPE=0 is set in the environment, run
- *     the two-phase kernel (USAGI_BSA_PIPE=1 makes every call without seq_lens on CSR or
- *     analytic rows use the pipelined one; read at each launch). Both meet the same parity
- *     bound; between them results can differ in the last bits.
+ *   - Kernel: chosen per call from the number of query blocks n = B*H*T/128 and the entries per
+ *     head (max_nnz, or the analytic pattern's own count). Few query blocks (n <= 128, n <= 256 with
+ *     rows of 6 blocks and more, n <= 512 with long rows that grow as full causal ones do) run
+ *     kernels that divide the keys of a block over the waves. Other calls without seq_lens whose
+ *     rows hold at most 4 key blocks on average (already from n = 64 on) run a software-pipelined
+ *     kernel, the rest the two-phase kernel. USAGI_BSA_PIPE=0 in the environment takes the
+ *     pipelined kernel out, USAGI_BSA_PIPE=1 makes every call without seq_lens on CSR or analytic
+ *     rows use it (read at each launch). All meet the same parity bound; between them results can
+ *     differ in the last bits.
  *   - Return: 0 on success; a negative USAGI_BSA_E* code for a rejected argument; a positive
  *     hipError_t value when the HIP runtime reports an error. usagi_bsa_last_error() gives a
  *     message for the calling thread's last failure.

@@ -16,7 +16,7 @@ REPO_DIR = os.path.dirname(PKG_DIR)
 INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 CSRC_DIR = os.path.join(PKG_DIR, "csrc")
 # The kernels and their launch ABI (HIP), and the host-only validator and work planner.
-SRCS = [os.path.join(CSRC_DIR, "bsa_fwd.hip"), os.path.join(CSRC_DIR, "bsa_plan.cpp")]
+SRCS = [os.path.join(CSRC_DIR, name) for name in ("bsa_fwd.hip", "bsa_ksplit.hip", "bsa_plan.cpp")]
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libusagi_bsa.so")
 ARCH = "gfx950"
@@ -40,6 +40,8 @@ def hipcc_command(srcs: list[str] | None = None, out: str = LIB_PATH,
         "-shared",
         # Packed FP32 VALU forms are kept out of the device code.
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        # MFMA accumulators stay in VGPRs while they fit, instead of being copied out of AGPRs.
+        "-mllvm", "-amdgpu-mfma-vgpr-form",
         "-I", INCLUDE_DIR,
         "-I", CSRC_DIR,
         *(extra or []),

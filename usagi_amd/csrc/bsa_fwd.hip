@@ -8,7 +8,8 @@
 // over fp32 scores scaled AFTER the dot product (v7:92, v7:96-100); P is rounded to fp16 before
 // P·V (v7:107). O = acc / l and LSE = m·ln2 + ln l (v7:138-148).
 //
-// One kernel template, bsa_fwd_dma_kernel<kBf16, kRows, kFullSeq>:
+// The kernel of large calls is one template, bsa_fwd_dma_kernel<kBf16, kRows, kFullSeq> (short rows:
+// bsa_fwd_pipe_kernel below; few query blocks: bsa_ksplit.hip; the choice: choose()):
 //   kBf16     fp16 or bf16 inputs (bf16: Q·K^T in bf16, V converted to fp16 in LDS, P·V in fp16
 //             as v7:107 does, O written in bf16).
 //   kRows     where a query block's key blocks come from: kRowsCsr (the v7 walk above),
@@ -52,124 +53,12 @@
 #include <type_traits>
 
 #include "usagi_bsa.h"
+#include "bsa_device.h"
 #include "bsa_internal.h"
 
 namespace {
 
-constexpr int kBlk = USAGI_BSA_BLOCK;    // rows per query / key block
-constexpr int kHd = USAGI_BSA_HEAD_DIM;  // head dimension
-constexpr int kThreads = 256;            // 4 wave64s
-constexpr float kLn2 = 0.6931471805599453f;
-constexpr float kSpecSum = 4096.0f;      // acceptance bound of a speculative P row sum
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-typedef _Float16 half2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-struct Args {
-  const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
-  uint16_t* o;
-  float* lse;
-  const int32_t* row_ptr;
-  const int32_t* col_idx;
-  const int32_t* seq_lens;
-  int heads;
-  int T;
-  int nqb;
-  int bh_count;
-  int max_nnz;
-  float qk_scale;  // log2(e) / sqrt(128)
-  int head_major;  // work-item order without a plan, see item_coords
-  int window;      // analytic rows (kRowsWindow): window length in blocks
-  int n_global;    // analytic rows: global prefix blocks
-  const int32_t* sched;  // planned order (usagi_bsa_plan): slot -> item, or NULL
-  int n_items;           // B * H * nqb
-};
-
-// Work item (workgroup index) -> (query block, b*h) when no plan is given.
-// head_major == 0: query blocks in descending order (for causal window patterns the longest
-//   rows first), b*h fastest.
-// head_major == 1 (B*H a multiple of 8): workgroups are dealt to the 8 XCDs round-robin by
-//   index, so item i runs on XCD i % 8; each XCD walks its heads x, x+8, ... one at a time, and
-//   within a head takes the query blocks in descending order. The key/value tiles of the head being
-//   walked (4 MiB at T = 8192) then stay in that XCD's L2 while all its query blocks read them.
-__device__ __forceinline__ void item_coords(const Args& a, int item, int& qb, int& bh) {
-  if (a.head_major) {
-    const int x = item & 7;
-    const int j = item >> 3;
-    const int hl = j / a.nqb;
-    qb = a.nqb - 1 - (j - hl * a.nqb);
-    bh = x + 8 * hl;
-  } else {
-    const int qslot = item / a.bh_count;
-    qb = a.nqb - 1 - qslot;
-    bh = item - qslot * a.bh_count;
-  }
-}
-
-__device__ __forceinline__ float wave_pair_max(float x) {
-  // {x[l], x[l ^ 32]} in some order; max is symmetric.
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-__device__ __forceinline__ float wave_pair_sum(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Max / sum over lanes l, l^16, l^32, l^48 (the four lane groups that hold one query row in the
-// 16x16 MFMA layouts): {x[l], x[l ^ 16]} then {y[l], y[l ^ 32]}, each in some order.
-__device__ __forceinline__ float wave_quad_max(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const float y = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  return wave_pair_max(y);
-}
-
-__device__ __forceinline__ float wave_quad_sum(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const float y = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  return wave_pair_sum(y);
-}
-
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// Two bf16 (one dword) -> two fp16 (one dword), round to nearest even: each bf16 widens exactly
-// to fp32 (its bits in the upper half), then one v_cvt_pk_f16_f32 packs the pair.
-__device__ __forceinline__ uint32_t bf16x2_to_f16x2(uint32_t w) {
-  const float lo = __uint_as_float(w << 16);
-  const float hi = __uint_as_float(w & 0xffff0000u);
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, half2));
-}
-// Two fp32 -> one dword of two fp16 / bf16 (v_cvt_pk_*_f32, round to nearest even). O is
-// rounded twice, to fp32 by the multiply with 1/l and then to the output type, as the reference's
-// fp32 division and cast do.
-template <bool kBf16>
-__device__ __forceinline__ uint32_t pack_out(float x, float y) {
-  if constexpr (kBf16) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{x, y}, bf16x2));
-  } else {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{x, y}, half2));
-  }
-}
-
-template <bool kBf16>
-__device__ __forceinline__ floatx4 mfma_qk16(u32x4 a, u32x4 b, floatx4 c) {
-  if constexpr (kBf16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a),
-                                                  __builtin_bit_cast(half8, b), c, 0, 0, 0);
-  }
-}
+using namespace usagi_bsa;
 
 // ---------------------------------------------------------------------------------------------
 // DMA kernel (fp16; bf16 with the V tile turned into fp16 in LDS): K and V tiles go HBM -> LDS by
@@ -193,69 +82,6 @@ __device__ __forceinline__ floatx4 mfma_qk16(u32x4 a, u32x4 b, floatx4 c) {
 // A 16-byte-per-lane LDS DMA holds the issuing wave for tens of cycles, so the eight 1 KiB
 // pieces of a wave's share are interleaved with MFMAs instead of being issued back to back.
 // ---------------------------------------------------------------------------------------------
-
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_cvoid;
-
-// One 16-byte-per-lane DMA: global (uniform base + per-lane byte offset) -> LDS at the uniform
-// byte address lds_addr + 16 * lane. Issued as inline asm so that the compiler's wait-count pass
-// does not treat it as aliasing every later LDS read; the kernel waits for it explicitly
-// (s_waitcnt vmcnt + s_barrier) before any wave reads the tile.
-template <int kImm>
-__device__ __forceinline__ void dma_16b(const void* gbase, uint32_t voff, uint32_t lds_addr) {
-  // M0 holds the LDS destination. It is listed as clobbered, but the compiler does not preserve
-  // a reserved register across an asm statement; this is safe because nothing else in the
-  // kernel uses M0 (tests/test_device_code.py checks the assembly for that).
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2 offset:%3"
-      :
-      : "s"(lds_addr), "v"(voff), "s"(gbase), "i"(kImm)
-      : "memory", "m0");
-}
-
-// 8 DMAs of one wave's 8 KiB share of a tile: instruction i moves row group i (1 KiB). The
-// instruction's immediate offset moves both the global and the LDS address, so 1024 (i % 4) goes
-// there and i >= 4 use global and LDS bases 4096 bytes further on.
-__device__ __forceinline__ void dma_tile8(const char* src, const uint32_t off[4], uint32_t lds) {
-  const char* src_hi = src + 4096;
-  const uint32_t lds_hi = lds + 4096;
-  dma_16b<0>(src, off[0], lds);
-  dma_16b<1024>(src, off[1], lds);
-  dma_16b<2048>(src, off[2], lds);
-  dma_16b<3072>(src, off[3], lds);
-  dma_16b<0>(src_hi, off[0], lds_hi);
-  dma_16b<1024>(src_hi, off[1], lds_hi);
-  dma_16b<2048>(src_hi, off[2], lds_hi);
-  dma_16b<3072>(src_hi, off[3], lds_hi);
-}
-
-__device__ __forceinline__ uint32_t lds_addr_of(const void* p) {
-  return (uint32_t)(uintptr_t)(lds_void*)p;
-}
-
-#define USAGI_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
-#define USAGI_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
-#define USAGI_FENCE() __builtin_amdgcn_sched_barrier(0)
-
-// Rows of one query block (kRows):
-//   kRowsCsr     the CSR walk of kernels/v7_blockptr_warpspec.py:77-136: entries before the last
-//                are attended unmasked, the last entry stands for the diagonal, which is taken
-//                implicitly as kb = qb and causally masked.
-//   kRowsWindow  analytic rows instead of the CSR (no row_ptr / col_idx reads): query block qb
-//                attends the global prefix 0 .. n_global-1 and the window max(0, qb-window+1) ..
-//                qb, deduplicated and ascending, the rows of kernels/v1_baseline.py:141-322
-//                (_fwd_window, _fwd_window_global).
-//   kRowsGeneric the generic CSR walk of kernels/v1_baseline.py:331-406: every entry of the row,
-//                in any order; an entry equal to qb takes the causal mask, keys at or past
-//                seq_len are masked, and a row without the diagonal does not attend it (an empty
-//                row gives O = 0, LSE = -inf). The first entry equal to qb is walked first.
-// kFullSeq: no seq_lens (every sequence has length T), so no query row or key is ever masked
-// by length and the masking code is compiled out.
-enum : int { kRowsCsr = 0, kRowsWindow = 1, kRowsGeneric = 2 };
 
 template <bool kBf16, int kRows, bool kFullSeq>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -1005,6 +831,7 @@ int prepare(Args& a, const void* q, const void* k, const void* v, const int32_t*
   a.n_global = 0;
   a.sched = nullptr;
   a.n_items = (int)(bh * nqb);
+  a.n_slots = a.n_items;
   return USAGI_BSA_OK;
 }
 
@@ -1023,6 +850,7 @@ int prepare_csr(Args& a, const int32_t* row_ptr, const int32_t* col_idx, int32_t
   a.col_idx = col_idx;
   a.max_nnz = max_nnz;
   a.sched = sched;
+  if (sched) a.n_slots = n_slots;
   return USAGI_BSA_OK;
 }
 
@@ -1043,19 +871,43 @@ LaunchEvents take_events() {
   return e;
 }
 
-// Which kernel runs a call without seq_lens on CSR or analytic rows: bsa_fwd_pipe_kernel
-// when the rows hold at most kPipeMaxBlocks key blocks on average (the diagonal included), else
-// bsa_fwd_dma_kernel. A CSR's column list holds max_nnz entries per (b, h), so its rows average
-// at most max_nnz / nqb blocks; analytic rows count their entries exactly, which gives the
-// same choice as the CSR walk of the same pattern.
-// With short rows a work item is mostly its fixed part (loads, the diagonal block, O), which the
-// pipelined kernel shortens; on longer rows both kernels end at the same speed, held by the
-// part's power limit (the pipelined loop's fewer cycles per block come with a lower clock).
-// USAGI_BSA_PIPE in the environment overrides the choice for such calls: "1" always the
+// Which kernel runs a call. Every rule goes by what the CSR walk and the analytic rows of the same
+// pattern both know (query blocks, entries per head), so that they make the same choice.
+//
+// Short rows: a call without seq_lens on CSR or analytic rows that hold at most kPipeMaxBlocks key
+// blocks on average (the diagonal included) runs bsa_fwd_pipe_kernel. A CSR's column list holds
+// max_nnz entries per (b, h), so its rows average at most max_nnz / nqb blocks; analytic rows count
+// their entries exactly. With short rows a work item is mostly its fixed part (loads, the diagonal
+// block, O), which the pipelined kernel shortens; on longer rows both kernels end at the same speed,
+// held by the part's power limit (the pipelined loop's fewer cycles per block come with a lower
+// clock). USAGI_BSA_PIPE in the environment overrides the choice for such calls: "1" always the
 // pipelined kernel, "0" never (read at every launch).
+//
+// Few query blocks: the kernels of bsa_ksplit.hip divide the keys of a block over the waves, which
+// shortens the chain of blocks of a row where the chip has room for more workgroups than there are
+// query blocks. Kernel times in us over a sliding window of w blocks (fp16 / bf16; dma:
+// bsa_fwd_dma_kernel, pipe: bsa_fwd_pipe_kernel, then 32, 64 and 128 query rows per workgroup):
+//   n = 48,  T 1024, w 2:  dma 9.0 / 9.7   pipe 7.6 / 8.9   32: 6.6 / 6.8
+//   n = 64,  T 1024, w 8:  dma 18.6 / 22.4                  32: 9.5 / 10.5   64: 13.5 / 15.8
+//   n = 96,  T 1024, w 8:  dma 19.1 / 22.6                  32: 13.6 / 14.5  64: 13.9 / 16.0
+//   n = 128, T 4096, w 16: dma 32.2 / 40.2                  32: 26.2 / 30.3  64: 21.0 / 25.4
+//   n = 256, T 4096, w 16: dma 32.4 / 40.1                  64: 40.8 / 48.7  128: 30.5 / 34.8
+//   n = 256, T 1024, w 4:  dma 12.6 / 14.4                                   128: 13.1 / 14.5
+// so the line to 32 rows lies at 64 query blocks (256 workgroups, one per CU), to 64 rows at 128
+// and to 128 rows at 256, the last only for rows of 6 blocks and more. Rows that grow towards the end
+// of the sequence leave the chip emptier still: full causal rows of 32 blocks take 36 (64 rows)
+// against 52 (128) at n = 160 and 44 against 52 at n = 256, and where two workgroups of
+// bsa_fwd_dma_kernel share a CU until the longest row ends (n = 512: 89 / 102 us), 72 / 79 with 128
+// rows; with equal rows (w 8 at n = 512) it is 33 against 40, the other way round, and with rows of 16
+// blocks at most 49 against 54.
 constexpr long long kPipeMaxBlocks = 4;
+constexpr int kSmall32 = 64;
+constexpr int kSmall64 = 128;
+constexpr int kSmall128 = 256;
+constexpr int kSmallCausal = 512;
 
-long long window_entries(const Args& a) {
+long long row_entries(const Args& a, int kRows) {
+  if (kRows != kRowsWindow) return a.max_nnz;
   long long n = 0;
   for (int qb = 0; qb < a.nqb; ++qb) {
     const int lo = qb - a.window + 1 > 0 ? qb - a.window + 1 : 0;
@@ -1064,21 +916,60 @@ long long window_entries(const Args& a) {
   return n;
 }
 
-bool use_pipe(const Args& a, int kRows) {
-  const char* e = getenv("USAGI_BSA_PIPE");
-  if (e && e[0] == '1') return true;
-  if (e && e[0] == '0') return false;
-  const long long entries = kRows == kRowsWindow ? window_entries(a) : (long long)a.max_nnz;
-  return entries <= kPipeMaxBlocks * a.nqb;
+// Longest row of the causal window that has this many entries per head (at most nqb): what equal
+// rows would need, given that row i cannot hold more than i + 1 blocks.
+double causal_row(long long entries, int nqb) {
+  const double b = 2.0 * nqb + 1.0;
+  const double d = b * b - 8.0 * (double)entries;
+  return d > 0.0 ? 0.5 * (b - sqrt(d)) : (double)nqb;
+}
+
+// Query rows per workgroup of the bsa_ksplit.hip kernel for this call, 0: none of them.
+int small_query_rows(const Args& a, int kRows, long long entries) {
+  if (a.n_items <= kSmall32) return 32;
+  if (a.n_items <= kSmall64) return 64;
+  if (a.n_items > kSmallCausal) return 0;
+  const double mean = (double)entries / a.nqb;
+  const double longest = kRows == kRowsGeneric ? mean : causal_row(entries, a.nqb);
+  if (a.n_items <= kSmall128) {
+    if (longest < 6.0) return 0;
+    return longest >= 1.75 * mean ? 64 : 128;
+  }
+  return mean >= 12.0 && longest >= 1.5 * mean ? 128 : 0;
+}
+
+struct Choice {
+  bool pipe;
+  int query_rows;  // bsa_ksplit.hip kernel, or 0
+};
+
+Choice choose(const Args& a, int kRows) {
+  const long long entries = row_entries(a, kRows);
+  if (kRows != kRowsGeneric && !a.seq_lens) {
+    const char* e = getenv("USAGI_BSA_PIPE");
+    if (e && e[0] == '1') return {true, 0};
+    // From 64 query blocks on short rows keep the pipelined kernel.
+    if (!(e && e[0] == '0') && entries <= kPipeMaxBlocks * a.nqb && a.n_items >= kSmall32) return {true, 0};
+  }
+  return {false, small_query_rows(a, kRows, entries)};
 }
 
 template <bool kBf16, int kRows>
-int launch(const Args& a, int slots, hipStream_t s, LaunchEvents ev) {
+int launch(const Args& a, hipStream_t s, LaunchEvents ev) {
   const void* fn = a.seq_lens
                        ? reinterpret_cast<const void*>(&bsa_fwd_dma_kernel<kBf16, kRows, false>)
                        : reinterpret_cast<const void*>(&bsa_fwd_dma_kernel<kBf16, kRows, true>);
+  const Choice c = choose(a, kRows);
   if constexpr (kRows == kRowsCsr || kRows == kRowsWindow) {
-    if (!a.seq_lens && use_pipe(a, kRows)) fn = reinterpret_cast<const void*>(&bsa_fwd_pipe_kernel<kRows, kBf16>);
+    if (c.pipe) fn = reinterpret_cast<const void*>(&bsa_fwd_pipe_kernel<kRows, kBf16>);
+  }
+  unsigned grid = (unsigned)a.n_slots;
+  unsigned threads = kThreads;
+  if (c.query_rows) {
+    const SmallKernel k = usagi_bsa_small_kernel(kBf16, kRows, c.query_rows);
+    fn = k.fn;
+    threads = k.threads;
+    grid = (unsigned)((a.n_slots + 7) / 8 * 8 * (kBlk / c.query_rows));
   }
   Args arg = a;
   void* params[] = {&arg};
@@ -1086,20 +977,20 @@ int launch(const Args& a, int slots, hipStream_t s, LaunchEvents ev) {
   // another HIP call is neither taken for it nor cleared).
   hipError_t err;
   if (ev.start || ev.stop) {
-    err = hipExtLaunchKernel(fn, dim3((unsigned)slots), dim3(kThreads), params, 0, s, ev.start,
+    err = hipExtLaunchKernel(fn, dim3(grid), dim3(threads), params, 0, s, ev.start,
                              ev.stop, 0);
   } else {
-    err = hipLaunchKernel(fn, dim3((unsigned)slots), dim3(kThreads), params, 0, s);
+    err = hipLaunchKernel(fn, dim3(grid), dim3(threads), params, 0, s);
   }
   if (err != hipSuccess) return usagi_bsa_fail((int)err, "kernel launch failed: %s", hipGetErrorString(err));
   return USAGI_BSA_OK;
 }
 
 template <int kRows>
-int launch_dtype(const Args& a, int32_t dtype, int slots, void* stream, LaunchEvents ev) {
+int launch_dtype(const Args& a, int32_t dtype, void* stream, LaunchEvents ev) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == USAGI_BSA_BF16 ? launch<true, kRows>(a, slots, s, ev)
-                                 : launch<false, kRows>(a, slots, s, ev);
+  return dtype == USAGI_BSA_BF16 ? launch<true, kRows>(a, s, ev)
+                                 : launch<false, kRows>(a, s, ev);
 }
 
 }  // namespace
@@ -1123,7 +1014,7 @@ extern "C" int usagi_bsa_fwd(const void* q, const void* k, const void* v,
   int rc = prepare(a, q, k, v, seq_lens, out, lse, batch, heads, seq_len, head_dim, dtype);
   if (rc == USAGI_BSA_OK) rc = prepare_csr(a, row_ptr, col_idx, max_nnz, sched, n_slots);
   if (rc != USAGI_BSA_OK) return rc;
-  return launch_dtype<kRowsCsr>(a, dtype, sched ? n_slots : a.n_items, stream, ev);
+  return launch_dtype<kRowsCsr>(a, dtype, stream, ev);
 }
 
 extern "C" int usagi_bsa_fwd_generic(const void* q, const void* k, const void* v,
@@ -1138,7 +1029,7 @@ extern "C" int usagi_bsa_fwd_generic(const void* q, const void* k, const void* v
   int rc = prepare(a, q, k, v, seq_lens, out, lse, batch, heads, seq_len, head_dim, dtype);
   if (rc == USAGI_BSA_OK) rc = prepare_csr(a, row_ptr, col_idx, max_nnz, sched, n_slots);
   if (rc != USAGI_BSA_OK) return rc;
-  return launch_dtype<kRowsGeneric>(a, dtype, sched ? n_slots : a.n_items, stream, ev);
+  return launch_dtype<kRowsGeneric>(a, dtype, stream, ev);
 }
 
 extern "C" int usagi_bsa_fwd_window(const void* q, const void* k, const void* v,
@@ -1155,5 +1046,5 @@ extern "C" int usagi_bsa_fwd_window(const void* q, const void* k, const void* v,
   if (n_global < 0) return usagi_bsa_fail(USAGI_BSA_EINVAL, "n_global must be >= 0, got %d", (int)n_global);
   a.window = window;
   a.n_global = n_global;
-  return launch_dtype<kRowsWindow>(a, dtype, a.n_items, stream, ev);
+  return launch_dtype<kRowsWindow>(a, dtype, stream, ev);
 }
