@@ -666,8 +666,8 @@ def main() -> int:
                            "cached_call_ms": round(float(np.median(t_hit)), 4)}
         submission.clear_csr_cache()
         first["note"] = ("host wall time of one call, synchronised before and after, median of "
-                         "5: first_call_ms with freshly cloned CSR tensors (cache miss: host copy, "
-                         "check, window pattern and plan before the launch), "
+                         "5: first_call_ms with freshly cloned CSR tensors (cache miss: check and "
+                         "window pattern on the GPU ahead of the launch, plan behind it), "
                          "first_call_unchecked_ms the same with USAGI_BSA_VALIDATE=0 (no check, no "
                          "synchronisation: the CSR walk launches at once and the host copy "
                          "follows it on the stream), cached_call_ms with the bench's own CSR "

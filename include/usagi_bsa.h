@@ -113,6 +113,21 @@ int usagi_bsa_fwd_window(const void* q, const void* k, const void* v,
 int usagi_bsa_check_csr(const int32_t* row_ptr, const int32_t* col_idx, const int32_t* seq_lens,
                         int32_t batch, int32_t heads, int32_t num_q_blocks, int32_t max_nnz);
 
+/* The same preconditions checked on the GPU, asynchronously on the stream, over DEVICE row_ptr /
+ * col_idx (no counterpart in the reference), for every row (no seq_lens), together with the window
+ * pattern and the length of the rows. result: int32 memory the GPU can write (pinned host memory, or
+ * device memory), result_cap >= USAGI_BSA_CHECK_CAP(B*H*num_q_blocks) values; num_q_blocks <=
+ * USAGI_BSA_CHECK_MAX_BLOCKS. Returns the number g > 0 of flag words, or a negative status (below
+ * -1000: -1000 - hipError_t of the launch). Once the kernel is done, of result: [0 .. g) flags (bit 0
+ * in any word: some row breaks a precondition, see usagi_bsa_check_csr for which; bit 1 in any word:
+ * the rows are not exactly the analytic rows of (window, n_global)), [g] window, [g+1] n_global,
+ * [g+2 ..] the entries of each row, b*H*nqb + h*nqb + qb. */
+#define USAGI_BSA_CHECK_MAX_BLOCKS 8192
+#define USAGI_BSA_CHECK_CAP(n_rows) ((int64_t)(n_rows) + 1024 + 2)
+int usagi_bsa_check_csr_gpu(const int32_t* row_ptr, const int32_t* col_idx, int32_t batch,
+                            int32_t heads, int32_t num_q_blocks, int32_t max_nnz, int32_t* result,
+                            int32_t result_cap, void* stream);
+
 /* Work plan over a HOST copy of row_ptr; no counterpart in the reference, whose grid is
  * (nqb, B*H) in index order (kernels/v7_blockptr_warpspec.py:178-179). When rows of different
  * heads differ in length, it spreads the work evenly over the GPU's 8 XCDs (each XCD on a few

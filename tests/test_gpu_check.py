@@ -1,0 +1,126 @@
+"""The CSR check on the GPU against the host check, window_pattern and the CSR itself: valid rows,
+rows broken in each way the host check names, window and near-window patterns, rows longer than a
+wave, few and many rows per wave; and the first call of the shim around it."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from tests._helpers import assert_close
+from oracle import c_ref
+from usagi_amd import _native, block_sparse_attn_fwd, submission
+from usagi_amd import patterns as P
+
+pytestmark = pytest.mark.gpu
+
+
+def gpu_check(rp, ci):
+    B, H, n1 = rp.shape
+    rows = B * H * (n1 - 1)
+    drp, dci = torch.from_numpy(rp).cuda(), torch.from_numpy(ci).cuda()
+    result = torch.empty(_native.check_cap(rows), dtype=torch.int32, pin_memory=True)
+    n = _native.check_csr_gpu(drp.data_ptr(), dci.data_ptr(), B, H, n1 - 1, ci.shape[-1],
+                              result.data_ptr(), result.numel(),
+                              torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    r = result.numpy()
+    flags = int(np.bitwise_or.reduce(r[:n]))
+    window = None if flags & 2 else (int(r[n]), int(r[n + 1]))
+    return bool(flags & 1), window, r[n + 2:n + 2 + rows].reshape(B, H, n1 - 1).copy()
+
+
+def host_check(rp, ci):
+    B, H, n1 = rp.shape
+    try:
+        _native.check_csr_host(rp, ci, B, H, n1 - 1, ci.shape[-1])
+    except ValueError:
+        return True
+    return False
+
+
+@pytest.mark.parametrize("B,H,T,w,g", [(1, 1, 128, 1, 0), (1, 3, 384, 2, 0), (2, 4, 1024, 3, 2),
+                                       (1, 2, 12800, 70, 5), (1, 1, 8192, 100, 0), (3, 40, 2560, 4, 0),
+                                       (1, 2, 1024, 2, 9)])
+def test_window_patterns(B, H, T, w, g):
+    rp, ci = P.global_csr(B, H, T, g, w) if g else P.sliding_csr(B, H, T, w)
+    print(f"case check window B{B} H{H} T{T} w{w} g{g}", flush=True)
+    bad, window, counts = gpu_check(rp, ci)
+    assert not bad and window == submission.window_pattern(rp, ci, T // 128)
+    assert np.array_equal(counts, np.diff(rp, axis=-1))
+    # one entry changed in the last head: a valid row or not, never the pattern
+    if T > 256:
+        rp2, ci2 = rp.copy(), ci.copy()
+        at = rp2[-1, -1, T // 128 - 1]
+        ci2[-1, -1, at] = (ci2[-1, -1, at] + 1) % (T // 128)
+        bad, window, _ = gpu_check(rp2, ci2)
+        assert bad == host_check(rp2, ci2)
+        assert window == submission.window_pattern(rp2, ci2, T // 128)
+
+
+def broken(rp, ci, how, rng):
+    b, h = rng.integers(0, rp.shape[0]), rng.integers(0, rp.shape[1])
+    qb = int(rng.integers(2, rp.shape[2] - 1))
+    rs, re = rp[b, h, qb], rp[b, h, qb + 1]
+    if how == "not diagonal":
+        ci[b, h, re - 1] = qb - 1
+    elif how == "above":
+        ci[b, h, rs] = qb
+    elif how == "negative":
+        ci[b, h, rs] = -3
+    elif how == "twice":
+        ci[b, h, re - 2] = ci[b, h, rs]
+    elif how == "empty":
+        rp[b, h, qb + 1] = rs
+    elif how == "past the list":
+        rp[b, h, -1] = ci.shape[-1] + 1
+    elif how == "start":
+        rp[b, h, 0] = 1
+
+
+@pytest.mark.parametrize("how", ["none", "not diagonal", "above", "negative", "twice", "empty",
+                                 "past the list", "start"])
+@pytest.mark.parametrize("B,H,T", [(1, 2, 2048), (2, 3, 12800), (1, 64, 4096)])
+def test_rows_against_the_host_check(B, H, T, how):
+    nqb = T // 128
+    rng = np.random.default_rng(nqb)
+
+    def row(b, h, i):  # entries before the diagonal in any order, at least two where there are two
+        n = min(i, int(rng.integers(2, 80)))
+        return [int(x) for x in rng.permutation(i)[:n]] + [i]
+
+    rp, ci = P.make_csr(B, H, T, row)
+    if how != "none":
+        broken(rp, ci, how, rng)
+    print(f"case check rows B{B} H{H} T{T} {how}", flush=True)
+    bad, window, counts = gpu_check(rp, ci)
+    assert bad == host_check(rp, ci) == (how != "none")
+    assert window == submission.window_pattern(rp, ci, nqb)
+    assert np.array_equal(counts, np.maximum(np.diff(rp, axis=-1), 0))
+
+
+@pytest.mark.parametrize("pad", [0, 700])
+def test_first_call_equals_later_calls(pad):
+    """The first call launches before the check's result is known; a window-shaped CSR (also one
+    with a padded column list) gives the same bits in every call, and a broken one raises."""
+    submission.clear_csr_cache()
+    B, H, T = 1, 8, 4096
+    rp, ci = P.sliding_csr(B, H, T, 4)
+    ci = np.concatenate([ci, np.zeros((B, H, pad), np.int32)], axis=-1)
+    q, k, v = P.make_qkv(B, H, T, seed=5)
+    dev = [x.cuda() for x in (q, k, v)] + [torch.from_numpy(x).cuda() for x in (rp, ci)]
+    print(f"case first call pad {pad}", flush=True)
+    o1, l1 = block_sparse_attn_fwd(*dev, None)
+    (entry,) = submission._csr_cache.values()
+    assert entry.window == (4, 0)
+    o2, l2 = block_sparse_attn_fwd(*dev, None)
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2) and torch.equal(l1, l2)
+    oo, _ = c_ref.fwd(q.float().numpy(), k.float().numpy(), v.float().numpy(), rp, ci, None,
+                      round_p_fp16=False)
+    assert_close(o1.float().cpu().numpy(), oo)
+    dev[4][0, 3, 9] = 31
+    with pytest.raises(ValueError, match="h=3"):
+        block_sparse_attn_fwd(*dev, None)
+    submission.clear_csr_cache()

@@ -21,6 +21,7 @@ EXPORTED_SYMBOLS = (
     "usagi_bsa_fwd_generic",
     "usagi_bsa_fwd_window",
     "usagi_bsa_check_csr",
+    "usagi_bsa_check_csr_gpu",
     "usagi_bsa_plan",
     "usagi_bsa_time_next_launch",
     "usagi_bsa_version",
@@ -58,6 +59,8 @@ def load() -> ctypes.CDLL:
     lib.usagi_bsa_fwd_window.restype = ctypes.c_int
     lib.usagi_bsa_check_csr.argtypes = [p, p, p, i32, i32, i32, i32]
     lib.usagi_bsa_check_csr.restype = ctypes.c_int
+    lib.usagi_bsa_check_csr_gpu.argtypes = [p, p, i32, i32, i32, i32, p, i32, p]
+    lib.usagi_bsa_check_csr_gpu.restype = ctypes.c_int
     lib.usagi_bsa_plan.argtypes = [p, i32, i32, i32, i32, p, i32]
     lib.usagi_bsa_plan.restype = ctypes.c_int
     lib.usagi_bsa_time_next_launch.argtypes = [p, p]
@@ -124,6 +127,25 @@ def plan_host(row_ptr, batch: int, heads: int, nqb: int, generic: bool = False):
     if n < 0:
         raise NativeError(n, last_error())
     return sched[:n].copy() if n else None
+
+
+# USAGI_BSA_CHECK_MAX_BLOCKS of include/usagi_bsa.h
+CHECK_MAX_BLOCKS = 8192
+
+
+def check_cap(n_rows: int) -> int:
+    """USAGI_BSA_CHECK_CAP of include/usagi_bsa.h."""
+    return n_rows + 1024 + 2
+
+
+def check_csr_gpu(row_ptr_ptr, col_idx_ptr, batch, heads, nqb, max_nnz, result_ptr, result_cap,
+                  stream) -> int:
+    """Launch the CSR check on the GPU; returns the number of flag words in the result."""
+    n = load().usagi_bsa_check_csr_gpu(row_ptr_ptr, col_idx_ptr, batch, heads, nqb, max_nnz,
+                                       result_ptr, result_cap, stream)
+    if n <= 0:
+        raise NativeError(n, last_error())
+    return n
 
 
 def check_csr_host(row_ptr, col_idx, batch: int, heads: int, nqb: int, max_nnz: int,

@@ -15,8 +15,10 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
 INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 CSRC_DIR = os.path.join(PKG_DIR, "csrc")
-# The kernels and their launch ABI (HIP), and the host-only validator and work planner.
-SRCS = [os.path.join(CSRC_DIR, name) for name in ("bsa_fwd.hip", "bsa_ksplit.hip", "bsa_plan.cpp")]
+# The kernels and their launch ABI (HIP), the CSR check on the GPU, and the host-only validator and
+# work planner.
+SRCS = [os.path.join(CSRC_DIR, name) for name in ("bsa_fwd.hip", "bsa_ksplit.hip", "bsa_check.hip",
+                                                 "bsa_plan.cpp")]
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libusagi_bsa.so")
 ARCH = "gfx950"

@@ -13,14 +13,16 @@ Differences from the reference, all deliberate:
     kernels/v7_blockptr_warpspec.py:107).
   * The launch goes through the C ABI of libusagi_bsa.so (compiled ahead of time for gfx950)
     instead of a Triton JIT launch.
-  * The first call with a given pair of CSR tensors copies them to the host once (one
-    synchronisation), checks every row (block_sparse_attn_fwd raises ValueError on a row that
-    is empty, repeats a block, lists a block outside [0, qb) before its last entry, or does not
-    end with its diagonal: the reference's walk, kernels/v7_blockptr_warpspec.py:83-111, would
-    silently attend future tokens or count a block twice there; the entries before the diagonal
+  * The first call with a given pair of CSR tensors checks every row on the GPU, ahead of the
+    forward kernel, and waits for the result while that one runs (CSR tensors on the host, and a
+    CSR that the GPU check rejects, are checked on the host). block_sparse_attn_fwd raises
+    ValueError on a row that is empty, repeats a block, lists a block outside [0, qb) before its
+    last entry, or does not end with its diagonal (the reference's walk,
+    kernels/v7_blockptr_warpspec.py:83-111, would silently attend future tokens or count a block
+    twice there; the entries before the diagonal
     may come in any order; rows of query blocks at or past seq_len, which the walk never reads
-    (v7:63-67), may hold anything) and plans the work order over the GPU. Later calls with the
-    same tensor objects, unmodified, reuse that (the reference memoises converted metadata on
+    (v7:63-67), may hold anything). The same call plans the work order of more than 256 query
+    blocks. Later calls with the same tensor objects, unmodified, reuse that (the reference memoises converted metadata on
     data_ptr() alone, kernels/v7_blockptr_warpspec.py:167-176; here the key also holds the
     shapes, dtypes, torch's in-place version counters and the tensor objects themselves, and,
     for a CSR that is only valid before seq_len, the seq_lens it was checked with). A CSR
@@ -64,6 +66,9 @@ _DTYPE_CODES = {torch.float16: _native.FP16, torch.bfloat16: _native.BF16}
 
 _CSR_CACHE_SIZE = 64
 
+# Query blocks up to which no work plan is made: they all run at once (one workgroup per CU or more).
+_PLAN_ITEMS = 256
+
 
 class _CsrEntry:
     """What the first call learnt about one (row_ptr, col_idx) pair: the tensors it was made
@@ -73,7 +78,7 @@ class _CsrEntry:
     checked with (seq_key; None: every row is valid)."""
 
     __slots__ = ("row_ptr", "col_idx", "sched", "n_slots", "stream", "window", "seq_key",
-                 "seq_ref", "pending", "sched_host", "sched_ready")
+                 "seq_ref", "pending", "sched_host", "sched_ready", "unchecked")
 
     def __init__(self, row_ptr, col_idx, sched, n_slots, stream, window, seq_key, seq_ref):
         self.row_ptr = weakref.ref(row_ptr)
@@ -91,6 +96,9 @@ class _CsrEntry:
         # Event after an asynchronous copy of the plan to the device (or None: the copy was
         # synchronous); a launch on another stream waits for it.
         self.sched_ready = None
+        # The key of an entry that is not in the cache yet (else None): the call that made it checks
+        # the CSR on the GPU (_start_check, _finish_check) around its launch.
+        self.unchecked = None
 
 
 _csr_cache: "OrderedDict[tuple, _CsrEntry]" = OrderedDict()
@@ -186,47 +194,114 @@ def _csr_entry(row_ptr, col_idx, B, H, nqb, dev, generic: bool, seq_lens=None) -
         done.record(stream)
         e = _CsrEntry(row_ptr, col_idx, None, 0, stream, None, None, None)
         e.pending = (done, rp_h, ci_h, B, H, nqb)
+    elif _on_gpu(row_ptr, col_idx, dev, nqb, max_nnz):
+        e = _CsrEntry(row_ptr, col_idx, None, 0, stream, None, None, None)
+        if not generic or B * H * nqb > _PLAN_ITEMS:
+            e.unchecked = key
+            return e
     else:
-        rp = row_ptr.detach().reshape(B, H, nqb + 1).to("cpu", torch.int32).contiguous().numpy()
-        ci = col_idx.detach().reshape(B, H, max_nnz).to("cpu", torch.int32).contiguous().numpy()
-        seq_key = seq_ref = None
-        if not generic and VALIDATE_CSR:
-            try:
-                _native.check_csr_host(rp, ci, B, H, nqb, max_nnz)
-            except ValueError:
-                # Rows past seq_len are never read, so they may hold anything: check the rest.
-                if seq_lens is None:
-                    raise
-                sl = torch.as_tensor(seq_lens).detach().to("cpu", torch.int32).reshape(-1).numpy()
-                _native.check_csr_host(rp, ci, B, H, nqb, max_nnz, seq_lens=sl)
-                seq_key, sref = _seq_key(seq_lens)
-                seq_ref = None if sref is None else weakref.ref(sref)
-        e = _CsrEntry(row_ptr, col_idx, None, 0, stream, None, seq_key, seq_ref)
-        _plan_entry(e, rp, ci, B, H, nqb, dev, generic)
+        e = _CsrEntry(row_ptr, col_idx, None, 0, stream, None, None, None)
+        _check_on_host(e, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
+    _remember(e, key)
+    return e
+
+
+def _remember(e: _CsrEntry, key: tuple) -> None:
     _csr_cache[key] = e
     while len(_csr_cache) > _CSR_CACHE_SIZE:
         _csr_cache.popitem(last=False)
-    return e
+
+
+def _on_gpu(row_ptr, col_idx, dev, nqb: int, max_nnz: int) -> bool:
+    """Whether the CSR can be checked on the GPU: there already, and not under stream capture (the
+    result is waited for)."""
+    return (dev.type == "cuda" and row_ptr.device == dev and col_idx.device == dev and max_nnz > 0
+            and nqb <= _native.CHECK_MAX_BLOCKS and not torch.cuda.is_current_stream_capturing())
+
+
+def _check_on_host(e: _CsrEntry, row_ptr, col_idx, B, H, nqb, dev, generic: bool, seq_lens) -> None:
+    """Check, window pattern and plan over host copies of the CSR; raises ValueError on a row that
+    the walk would misread."""
+    max_nnz = col_idx.shape[-1] if col_idx.dim() else 0
+    rp = row_ptr.detach().reshape(B, H, nqb + 1).to("cpu", torch.int32).contiguous().numpy()
+    ci = col_idx.detach().reshape(B, H, max_nnz).to("cpu", torch.int32).contiguous().numpy()
+    if not generic and VALIDATE_CSR:
+        try:
+            _native.check_csr_host(rp, ci, B, H, nqb, max_nnz)
+        except ValueError:
+            # Rows past seq_len are never read, so they may hold anything: check the rest.
+            if seq_lens is None:
+                raise
+            sl = torch.as_tensor(seq_lens).detach().to("cpu", torch.int32).reshape(-1).numpy()
+            _native.check_csr_host(rp, ci, B, H, nqb, max_nnz, seq_lens=sl)
+            e.seq_key, sref = _seq_key(seq_lens)
+            e.seq_ref = None if sref is None else weakref.ref(sref)
+    _plan_entry(e, rp, ci, B, H, nqb, dev, generic)
+
+
+def _start_check(rp, ci, B, H, nqb, max_nnz, stream) -> tuple:
+    """Launch the GPU check of int32 device tensors; the forward launch follows it on the stream."""
+    cap = _native.check_cap(B * H * nqb)
+    result = torch.empty(cap, dtype=torch.int32, pin_memory=True)
+    n_flags = _native.check_csr_gpu(rp.data_ptr(), ci.data_ptr(), B, H, nqb, max_nnz,
+                                    result.data_ptr(), cap, stream.cuda_stream)
+    done = torch.cuda.Event()
+    done.record(stream)
+    return done, result, n_flags
+
+
+def _finish_check(e: _CsrEntry, check: tuple, row_ptr, col_idx, B, H, nqb, dev, generic: bool,
+                  seq_lens) -> int:
+    """Wait for the check (the forward kernel is queued behind it or running), keep what it found in
+    the entry and the entry in the cache; a CSR that it rejects is looked at again on the host, which
+    raises with the row's position or accepts the rows before seq_len. Returns the entries of the
+    first head."""
+    import numpy as np
+
+    done, result, n_flags = check
+    done.synchronize()
+    r = result.numpy()
+    flags = int(np.bitwise_or.reduce(r[:n_flags]))
+    key, e.unchecked = e.unchecked, None
+    if flags & 1 and not generic:
+        _check_on_host(e, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
+    else:
+        rows = B * H * nqb
+        if rows > _PLAN_ITEMS:
+            rp = np.zeros((B * H, nqb + 1), dtype=np.int32)
+            np.cumsum(r[n_flags + 2:n_flags + 2 + rows].reshape(B * H, nqb), axis=1, out=rp[:, 1:])
+            _plan_rows(e, rp, B, H, nqb, dev, generic, pinned=True)
+        if not generic and ROUTE_WINDOW and not flags & 2 and e.sched is None:
+            e.window = (int(r[n_flags]), int(r[n_flags + 1]))
+    _remember(e, key)
+    return int(r[n_flags + 2:n_flags + 2 + nqb].sum())
+
+
+def _plan_rows(e: _CsrEntry, rp, B, H, nqb, dev, generic: bool, pinned=False) -> None:
+    """Work plan of a host row_ptr, into the entry. With at most _PLAN_ITEMS query blocks every
+    workgroup runs at once and the order does not matter."""
+    if B * H * nqb <= _PLAN_ITEMS:
+        return
+    sched = _native.plan_host(rp, B, H, nqb, generic)
+    if sched is None:
+        return
+    src = torch.from_numpy(sched)
+    if pinned:  # copied behind the stream's queued work, no synchronisation
+        src = src.pin_memory()
+        e.sched_host = src  # stays alive until the copy has run
+    e.sched = src.to(dev, non_blocking=pinned)
+    e.n_slots = len(sched)
+    e.stream = torch.cuda.current_stream(dev) if dev.type == "cuda" else None
+    if pinned:
+        e.sched_ready = torch.cuda.Event()
+        e.sched_ready.record(e.stream)
 
 
 def _plan_entry(e: _CsrEntry, rp, ci, B, H, nqb, dev, generic: bool, pinned=False) -> None:
     """Work plan and window pattern of a host copy of the CSR, into the entry."""
-    window = None
-    if not generic and ROUTE_WINDOW and ci.shape[-1]:
-        window = window_pattern(rp, ci, nqb)
-    sched = _native.plan_host(rp, B, H, nqb, generic)
-    if sched is not None:
-        src = torch.from_numpy(sched)
-        if pinned:  # copied behind the stream's queued work, no synchronisation
-            src = src.pin_memory()
-            e.sched_host = src  # stays alive until the copy has run
-        e.sched = src.to(dev, non_blocking=pinned)
-        e.n_slots = len(sched)
-        e.stream = torch.cuda.current_stream(dev) if dev.type == "cuda" else None
-        if pinned:
-            e.sched_ready = torch.cuda.Event()
-            e.sched_ready.record(e.stream)
-    e.window = window if sched is None else None
+    _plan_rows(e, rp, B, H, nqb, dev, generic, pinned)
+    if e.sched is None and not generic and ROUTE_WINDOW and ci.shape[-1]:
+        e.window = window_pattern(rp, ci, nqb)
 
 
 def _finish_pending(e: _CsrEntry, dev, generic: bool) -> None:
@@ -289,11 +364,15 @@ def _run_csr(q, k, v, row_ptr, col_idx, seq_lens, generic: bool):
     lse = torch.empty((B, H, T), device=dev, dtype=torch.float32)
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream(dev)
-        if plan.window is not None:
+
+        def launch_window():
             _native.fwd_window(q.data_ptr(), k.data_ptr(), v.data_ptr(), plan.window[0],
                                plan.window[1], sl.data_ptr() if sl is not None else None,
                                out.data_ptr(), lse.data_ptr(), B, H, T, D,
                                _DTYPE_CODES[q.dtype], stream.cuda_stream)
+
+        if plan.window is not None:
+            launch_window()
             return out, lse
         rp = _as_int32_device(row_ptr, dev, (B, H, nqb + 1))
         ci = _as_int32_device(col_idx, dev, (B, H, max_nnz))
@@ -304,11 +383,18 @@ def _run_csr(q, k, v, row_ptr, col_idx, seq_lens, generic: bool):
             if plan.sched_ready is not None:
                 stream.wait_event(plan.sched_ready)
             plan.sched.record_stream(stream)
+        check = _start_check(rp, ci, B, H, nqb, max_nnz, stream) if plan.unchecked is not None else None
         _native.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), rp.data_ptr(),
                     ci.data_ptr() if max_nnz else None, sl.data_ptr() if sl is not None else None,
                     out.data_ptr(), lse.data_ptr(), B, H, T, D, max_nnz, _DTYPE_CODES[q.dtype],
                     plan.sched.data_ptr() if plan.sched is not None else None, plan.n_slots,
                     stream.cuda_stream, generic=generic)
+        if check is not None:
+            entries = _finish_check(plan, check, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
+            if plan.window is not None and entries != max_nnz:
+                # A padded column list may have led to another kernel than the later calls' analytic
+                # rows, whose results differ in the last bits: this call gives theirs.
+                launch_window()
     return out, lse
 
 
