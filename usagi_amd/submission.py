@@ -43,6 +43,8 @@ Differences from the reference, all deliberate:
 
 from __future__ import annotations
 
+import contextlib
+import math
 import os
 import weakref
 from collections import OrderedDict
@@ -65,6 +67,11 @@ ROUTE_WINDOW = os.environ.get("USAGI_BSA_ROUTE_WINDOW", "1") not in ("", "0")
 _DTYPE_CODES = {torch.float16: _native.FP16, torch.bfloat16: _native.BF16}
 
 _CSR_CACHE_SIZE = 64
+
+# Handle of the current stream of a device (by index), as torch.cuda.current_stream().cuda_stream.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+_NOTHING = contextlib.nullcontext()
 
 # Query blocks up to which no work plan is made: they all run at once (one workgroup per CU or more).
 _PLAN_ITEMS = 256
@@ -113,7 +120,7 @@ def _tensor_key(t: torch.Tensor) -> tuple:
     # Inference tensors have no version counter: an in-place change to one made in inference
     # mode is not seen (like a change made outside torch, it needs clear_csr_cache()).
     version = None if t.is_inference() else t._version
-    return (t.device, t.data_ptr(), tuple(t.shape), tuple(t.stride()), t.dtype, version)
+    return (t.device, t.data_ptr(), t.shape, t.stride(), t.dtype, version)
 
 
 def _seq_key(seq_lens):
@@ -244,9 +251,9 @@ def _start_check(rp, ci, B, H, nqb, max_nnz, stream) -> tuple:
     cap = _native.check_cap(B * H * nqb)
     result = torch.empty(cap, dtype=torch.int32, pin_memory=True)
     n_flags = _native.check_csr_gpu(rp.data_ptr(), ci.data_ptr(), B, H, nqb, max_nnz,
-                                    result.data_ptr(), cap, stream.cuda_stream)
+                                    result.data_ptr(), cap, stream)
     done = torch.cuda.Event()
-    done.record(stream)
+    done.record()
     return done, result, n_flags
 
 
@@ -311,13 +318,34 @@ def _finish_pending(e: _CsrEntry, dev, generic: bool) -> None:
 
 
 def _as_int32_device(t: torch.Tensor, device: torch.device, shape: tuple) -> torch.Tensor:
+    """t's values as contiguous int32 on the device (in `shape`'s order; its own shape where it
+    already is that: only the memory is used)."""
+    if (t.dtype == torch.int32 and t.device == device and t.is_contiguous()
+            and t.numel() == math.prod(shape)):
+        return t
     t = t.reshape(shape)
     if t.device != device or t.dtype != torch.int32 or not t.is_contiguous():
         t = t.to(device=device, dtype=torch.int32).contiguous()
     return t
 
 
+def _on_device(dev: torch.device):
+    """Context in which dev is the current device (nothing to switch where it already is)."""
+    if dev.index == torch.cuda.current_device():
+        return _NOTHING
+    return torch.cuda.device(dev)
+
+
 def _check_inputs(q, k, v):
+    # What every good call passes first, in few attribute reads; anything else is named below.
+    if isinstance(q, torch.Tensor) and isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor):
+        shape, dtype, dev = q.shape, q.dtype, q.device
+        if (dev.type == "cuda" and dtype in _DTYPE_CODES and len(shape) == 4
+                and k.shape == shape and v.shape == shape and k.dtype == dtype
+                and v.dtype == dtype and k.device == dev and v.device == dev):
+            B, H, T, D = shape
+            if D == HEAD_DIM and T > 0 and T % BLOCK_SIZE == 0:
+                return B, H, T, D
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor")
@@ -362,33 +390,34 @@ def _run_csr(q, k, v, row_ptr, col_idx, seq_lens, generic: bool):
         sl = _as_int32_device(torch.as_tensor(seq_lens), dev, (B,))
     out = torch.empty((B, H, T, D), device=dev, dtype=q.dtype)
     lse = torch.empty((B, H, T), device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev)
+    with _on_device(dev):
+        stream = _raw_stream(dev.index)  # of torch's current stream; no Stream object per call
 
         def launch_window():
             _native.fwd_window(q.data_ptr(), k.data_ptr(), v.data_ptr(), plan.window[0],
                                plan.window[1], sl.data_ptr() if sl is not None else None,
                                out.data_ptr(), lse.data_ptr(), B, H, T, D,
-                               _DTYPE_CODES[q.dtype], stream.cuda_stream)
+                               _DTYPE_CODES[q.dtype], stream)
 
         if plan.window is not None:
             launch_window()
             return out, lse
         rp = _as_int32_device(row_ptr, dev, (B, H, nqb + 1))
         ci = _as_int32_device(col_idx, dev, (B, H, max_nnz))
-        if plan.sched is not None and stream != plan.stream:
+        if plan.sched is not None and stream != plan.stream.cuda_stream:
             # The plan's memory belongs to the stream it was copied on; a launch on another
             # stream waits for an asynchronous copy to land and keeps the memory from being
             # reused while the kernel reads it.
+            current = torch.cuda.current_stream(dev)
             if plan.sched_ready is not None:
-                stream.wait_event(plan.sched_ready)
-            plan.sched.record_stream(stream)
+                current.wait_event(plan.sched_ready)
+            plan.sched.record_stream(current)
         check = _start_check(rp, ci, B, H, nqb, max_nnz, stream) if plan.unchecked is not None else None
         _native.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), rp.data_ptr(),
                     ci.data_ptr() if max_nnz else None, sl.data_ptr() if sl is not None else None,
                     out.data_ptr(), lse.data_ptr(), B, H, T, D, max_nnz, _DTYPE_CODES[q.dtype],
                     plan.sched.data_ptr() if plan.sched is not None else None, plan.n_slots,
-                    stream.cuda_stream, generic=generic)
+                    stream, generic=generic)
         if check is not None:
             entries = _finish_check(plan, check, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
             if plan.window is not None and entries != max_nnz:
@@ -439,8 +468,8 @@ def block_sparse_attn_fwd_window(q, k, v, window, n_global=0, seq_lens=None):
         sl = _as_int32_device(torch.as_tensor(seq_lens), dev, (B,))
     out = torch.empty((B, H, T, D), device=dev, dtype=q.dtype)
     lse = torch.empty((B, H, T), device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with _on_device(dev):
+        stream = _raw_stream(dev.index)
         _native.fwd_window(q.data_ptr(), k.data_ptr(), v.data_ptr(), window, n_global,
                            sl.data_ptr() if sl is not None else None, out.data_ptr(),
                            lse.data_ptr(), B, H, T, D, _DTYPE_CODES[q.dtype], stream)
