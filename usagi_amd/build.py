@@ -44,6 +44,9 @@ def hipcc_command(srcs: list[str] | None = None, out: str = LIB_PATH,
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         # MFMA accumulators stay in VGPRs while they fit, instead of being copied out of AGPRs.
         "-mllvm", "-amdgpu-mfma-vgpr-form",
+        # The key loop of bsa_fwd_dma_kernel is instruction-fetch sensitive: started on a 64-byte line,
+        # rows of 80 bf16 blocks take 287 us instead of 305, retrieval rows 230 instead of 233.
+        "-falign-loops=64",
         "-I", INCLUDE_DIR,
         "-I", CSRC_DIR,
         *(extra or []),
