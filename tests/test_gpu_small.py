@@ -91,3 +91,27 @@ def test_scores_that_outgrow_the_running_max(H, T):
     k[:, :, 37:128] *= 6.0
     print(f"case small growth H{H} T{T}", flush=True)
     check(block_sparse_attn_fwd, rp, ci, q, k, v)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H", [2, 8, 40])  # n = 32, 128 and 640: bsa_ksplit.hip and bsa_fwd_dma_kernel
+def test_rows_past_seq_len_hold_anything(H, dtype):
+    """q, k and v past seq_len are NaN: the rows before it (seq_len a multiple of 32, the keys of a
+    P·V step) are those of clean inputs, the rows past it O = 0 and LSE = -inf."""
+    B, T, sl = 2, 1024, [608, 96]
+    rp, ci = P.sliding_csr(B, H, T, 3)
+    q, k, v = P.make_qkv(B, H, T, seed=H, dtype=dtype)
+    dirty = [x.clone() for x in (q, k, v)]
+    for x in dirty:
+        for b in range(B):
+            x[b, :, sl[b]:] = float("nan")
+    print(f"case dirty tail H{H} {dtype}", flush=True)
+    o, lse = block_sparse_attn_fwd(*(x.to(DEV) for x in dirty), torch.from_numpy(rp).to(DEV),
+                                   torch.from_numpy(ci).to(DEV),
+                                   torch.tensor(sl, dtype=torch.int32, device=DEV))
+    torch.cuda.synchronize()
+    oo, ol = c_ref.fwd(q.float().numpy(), k.float().numpy(), v.float().numpy(), rp, ci,
+                       np.asarray(sl, np.int32), round_p_fp16=False)
+    rtol = 2e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0)
+    assert_close(o.float().cpu().numpy(), oo, rtol=rtol)
+    assert_close(lse.cpu().numpy(), ol, what="LSE")

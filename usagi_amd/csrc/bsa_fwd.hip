@@ -163,13 +163,18 @@ void bsa_fwd_dma_kernel(Args a) {
     qvalid[qt] = kFullSeq || qrow[qt] < seq_len;
   }
 
-  // Q^T operands (MFMA B, 32 d x 16 queries): tile qt, k-step ks holds d = 32ks + 8g4 .. +7.
+  // Q^T operands (MFMA B, 32 d x 16 queries): tile qt, k-step ks holds d = 32ks + 8g4 .. +7. Rows past
+  // seq_len may hold anything: they are taken as zero, so that their scores are finite and need no
+  // mask in the key loop (their O and LSE are replaced in the epilogue).
   u32x4 qf[2][4];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     const uint16_t* qp = a.q + base + (size_t)qrow[qt] * kHd + 8 * g4;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = *(const u32x4*)(qp + 32 * ks);
+    for (int ks = 0; ks < 4; ++ks) {
+      const u32x4 x = *(const u32x4*)(qp + 32 * ks);
+      qf[qt][ks] = qvalid[qt] ? x : u32x4{0, 0, 0, 0};
+    }
   }
 
   const int nqb_m1 = a.nqb - 1;
@@ -294,13 +299,11 @@ void bsa_fwd_dma_kernel(Args a) {
   // real s_waitcnt so the compiler knows no load of its own is outstanding inside the loop.
   __builtin_amdgcn_s_waitcnt(0x0F70);
 
-  // One key block: the diagonal (kDiag, j = -1, causal mask) or off-diagonal entry j.
-  // kMaskQ: some query rows of this block may be past seq_len. kNext: DMA the K tile of entry
-  // j + 1 during this block's P·V. The generic walk masks off-diagonal entries by their key
+  // One key block: the diagonal (kDiag, j = -1, causal mask) or off-diagonal entry j. kNext: DMA
+  // the K tile of entry j + 1 during this block's P·V. The generic walk masks off-diagonal entries by their key
   // block: an entry equal to qb (a repeated diagonal) causally, one above qb by seq_len.
-  auto block = [&](auto diag_tag, auto maskq_tag, auto next_tag, int j) {
+  auto block = [&](auto diag_tag, auto next_tag, int j) {
     constexpr bool kDiag = decltype(diag_tag)::value;
-    constexpr bool kMaskQ = decltype(maskq_tag)::value;
     constexpr bool kNext = decltype(next_tag)::value;
     USAGI_WAIT_VM(0);  // this wave's K(j) DMA has landed
     USAGI_BARRIER();   // K(j) complete; every wave is done reading V of the previous block
@@ -368,10 +371,11 @@ void bsa_fwd_dma_kernel(Args a) {
           } else if (t == 2 * wave + qt) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              if (4 * g4 + r > c16 || !qvalid[qt]) st[qt][t][r] = -INFINITY;
+              if (4 * g4 + r > c16) st[qt][t][r] = -INFINITY;
             }
-          } else if (!qvalid[qt]) {
-            st[qt][t] = floatx4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+          }
+          if (!qvalid[qt] && t <= 2 * wave + qt) {
+            st[qt][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};  // K past seq_len may hold anything too
           }
         }
       }
@@ -395,15 +399,6 @@ void bsa_fwd_dma_kernel(Args a) {
                 if (16 * t + r > lim) st[qt][t][r] = -INFINITY;
               }
             }
-          }
-        }
-      }
-      if constexpr (kMaskQ) {
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-          if (!qvalid[qt]) {
-#pragma unroll
-            for (int t = 0; t < 8; ++t) st[qt][t] = floatx4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
           }
         }
       }
@@ -555,21 +550,17 @@ void bsa_fwd_dma_kernel(Args a) {
 
   using T_ = std::true_type;
   using F_ = std::false_type;
-  using MaskQ = std::integral_constant<bool, !kFullSeq>;
-  // With seq_lens, off-diagonal blocks use the kMaskQ form even when every query row of the
-  // block is valid (the masking branch is then skipped for the whole wave): separate full-block
-  // copies of the block body push the register allocation of the whole kernel into spills.
   // Generic rows without the diagonal start with an off-diagonal block from m = -1e30: its
   // speculative P overflows, so it takes the exact row max like any block that outgrows m.
   if (has_diag) {
     if (n_off > 0) {
-      block(T_{}, MaskQ{}, T_{}, -1);
+      block(T_{}, T_{}, -1);
     } else {
-      block(T_{}, MaskQ{}, F_{}, -1);
+      block(T_{}, F_{}, -1);
     }
   }
-  for (int j = 0; j < n_off - 1; ++j) block(F_{}, MaskQ{}, T_{}, j);
-  if (n_off > 0) block(F_{}, MaskQ{}, F_{}, n_off - 1);
+  for (int j = 0; j < n_off - 1; ++j) block(F_{}, T_{}, j);
+  if (n_off > 0) block(F_{}, F_{}, n_off - 1);
 
   float l_tot[2];
   float inv[2];
