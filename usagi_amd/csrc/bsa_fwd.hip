@@ -89,6 +89,12 @@ void bsa_fwd_dma_kernel(Args a) {
   __shared__ __attribute__((aligned(1024))) uint16_t k_lds[kBlk * kHd];  // K[key][d], swizzled
   __shared__ __attribute__((aligned(1024))) uint16_t v_lds[kBlk * kHd];  // V[key][d], swizzled
   constexpr bool kGeneric = kRows == kRowsGeneric;
+  // bf16 V on its way to fp16 in LDS: through registers (global load, convert, LDS write), which
+  // saves the DMA's LDS write and the conversion's LDS read, or in place after its DMA. Through
+  // registers is 1-3% faster on analytic rows (sliding w8 B2 H16 T8192: 142.5 against 145.0 us) and
+  // generic rows (128.4 against 131.6), but not on CSR rows (rows of 80 blocks, B1 H2 T32768: 290
+  // against 286), whose column registers leave the scheduler less room.
+  constexpr bool kVRegs = kBf16 && kRows != kRowsCsr;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -334,7 +340,16 @@ void bsa_fwd_dma_kernel(Args a) {
     for (int f = 0; f < 4; ++f) {
       if (k_needed(f)) kop[f] = k_read(f);
     }
-    // V(j) DMA pieces go out between the MFMAs (the V buffer is free after the barrier).
+    // V(j) DMA pieces go out between the MFMAs (the V buffer is free after the barrier). kVRegs: this
+    // wave's rows of V(j) come into registers instead.
+    u32x4 vreg[4];
+    const char* vrow_src = vt_src + wave * 8192 + lane * 16;
+    auto put_v = [&](int i) {  // rows 4i .. 4i+3 of the wave's, swizzled as the DMA writes them
+      u32x4 x = vreg[i & 3];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) x[w] = bf16x2_to_f16x2(x[w]);
+      *(u32x4*)((char*)v_lds + i * 1024 + v_off[i & 1]) = x;
+    };
 #pragma unroll
     for (int f = 0; f < 32; ++f) {
       const int t = f & 7;
@@ -345,7 +360,11 @@ void bsa_fwd_dma_kernel(Args a) {
       for (int qt = 0; qt < 2; ++qt) {
         if (!kDiag || t <= 2 * wave + qt) st[qt][t] = mfma_qk16<kBf16>(ka, qf[qt][ks], st[qt][t]);
       }
-      if ((f & 3) == 3) dma_piece(vt_src, v_off, v_dst, f >> 2);
+      if constexpr (kVRegs) {
+        if (f < 8 && (f & 1)) vreg[f >> 1] = *(const u32x4*)(vrow_src + (f >> 1) * 1024);
+      } else {
+        if ((f & 3) == 3) dma_piece(vt_src, v_off, v_dst, f >> 2);
+      }
     }
     // Schedule: the fragment four ahead is read before each pair of MFMAs.
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 1);
@@ -356,6 +375,13 @@ void bsa_fwd_dma_kernel(Args a) {
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 8, 1);
 
+    if constexpr (kVRegs) {
+      // Half of the rows at a time: 16 registers.
+#pragma unroll
+      for (int i = 0; i < 4; ++i) put_v(i);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vreg[i] = *(const u32x4*)(vrow_src + (4 + i) * 1024);
+    }
     // ---- masks (v7:94, v7:119-122), row max, speculative P. S^T tile t of query tile qt holds
     // keys 16t + 4g4 .. +3 of query row q_local[qt].
     if constexpr (kDiag) {
@@ -477,7 +503,10 @@ void bsa_fwd_dma_kernel(Args a) {
     l_part[1] += pblk[1];
 
     USAGI_WAIT_VM(0);  // V(j) has landed
-    if constexpr (kBf16) {
+    if constexpr (kVRegs) {
+#pragma unroll
+      for (int i = 4; i < 8; ++i) put_v(i);
+    } else if constexpr (kBf16) {
       // bf16 inputs: this wave turns its own 8 KiB of the V tile (the rows its DMA wrote) into
       // fp16 in place before the barrier publishes the tile, so P·V runs on fp16 P and fp16 V as
       // the reference's does (v7:107). Element positions do not matter: every 16-bit value is
