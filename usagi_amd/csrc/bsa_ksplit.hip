@@ -556,12 +556,30 @@ void bsa_wide_kernel(Args a) {
   uint32_t v_off[4];
   dma_offsets(lane, k_off, v_off);
   const uint32_t dst0 = __builtin_amdgcn_readfirstlane(lds_addr_of(lds) + wave * 4096);
+  // bf16: the rows of V come into registers and go to LDS as fp16 (put_v), swizzled as the DMA of
+  // fp16 inputs writes them, so that P·V runs on fp16 P and fp16 V.
+  u32x4 vreg[4];
+  auto load_v = [&](int kb, int i) {
+    vreg[i] = *(const u32x4*)(v_head + (size_t)kb * kTileBytes + i * 1024 + lane * 16);
+  };
+  auto put_v = [&](int stage, int i) {
+    u32x4 x = vreg[i];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) x[w] = bf16x2_to_f16x2(x[w]);
+    *(u32x4*)(lds + (2 * stage + 1) * kTileBytes + wave * 4096 + i * 1024 + v_off[i & 1]) = x;
+  };
   auto fetch = [&](int kb, int stage) {
     const uint32_t dst = dst0 + stage * 2 * kTileBytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i) dma_piece(k_head + (size_t)kb * kTileBytes, k_off, dst, i);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma_piece(v_head + (size_t)kb * kTileBytes, v_off, dst + kTileBytes, i);
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (kBf16) {
+        load_v(kb, i);
+      } else {
+        dma_piece(v_head + (size_t)kb * kTileBytes, v_off, dst + kTileBytes, i);
+      }
+    }
   };
 
   const int seq_len = a.seq_lens ? a.seq_lens[bh / a.heads] : a.T;
@@ -588,6 +606,12 @@ void bsa_wide_kernel(Args a) {
     if (n_blk > 0) fetch(row.key_block(0), 0);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);
+  if constexpr (kBf16) {
+    if (n_blk > 0) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) put_v(0, n);
+    }
+  }
 
   // Step i: the tiles of step i + 1 (kMore) are requested during Q·K^T into the other stage, whose
   // readers all passed this step's barrier.
@@ -600,21 +624,7 @@ void bsa_wide_kernel(Args a) {
     const char* k1 = k_head + (size_t)kb1 * kTileBytes;
     const char* v1 = v_head + (size_t)kb1 * kTileBytes;
     const uint32_t dst = dst0 + (stage ^ 1) * 2 * kTileBytes;
-    USAGI_WAIT_VM(0);  // this wave's rows of K(i) and V(i) have landed
-    if constexpr (kBf16) {
-      // Its rows of V(i) become fp16 in place, so that P·V runs on fp16 P and fp16 V.
-      char* slice = lds + (2 * stage + 1) * kTileBytes + wave * 4096 + lane * 16;
-      u32x4 x[4];
-#pragma unroll
-      for (int n = 0; n < 4; ++n) x[n] = *(const u32x4*)(slice + n * 1024);
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) x[n][w] = bf16x2_to_f16x2(x[n][w]);
-      }
-#pragma unroll
-      for (int n = 0; n < 4; ++n) *(u32x4*)(slice + n * 1024) = x[n];
-    }
+    USAGI_WAIT_VM(0);  // this wave's rows of K(i) and V(i) have landed (bf16: V(i) is in LDS as fp16)
     USAGI_BARRIER();
 
     // ---- S^T = K · Q^T: fragment f = kNT * ks + t, read four ahead.
@@ -646,7 +656,13 @@ void bsa_wide_kernel(Args a) {
         constexpr int kEvery = kF / 8;
         if (f % kEvery == kEvery - 1) {
           const int p = f / kEvery;
-          if (p < 4) {
+          if constexpr (kBf16) {
+            if (p < 4) {
+              load_v(kb1, p);
+            } else {
+              dma_piece(k1, k_off, dst, p - 4);
+            }
+          } else if (p < 4) {
             dma_piece(k1, k_off, dst, p);
           } else {
             dma_piece(v1, v_off, dst + kTileBytes, p - 4);
@@ -687,6 +703,9 @@ void bsa_wide_kernel(Args a) {
         for (int qt = 0; qt < 2; ++qt) {
           s.o[qt][g & 7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[qt][g >> 3], s.o[qt][g & 7], 0, 0, 0);
         }
+      }
+      if constexpr (kBf16 && kMore) {
+        if (g >= kG - 8 && g % 2 == 1) put_v(stage ^ 1, (g - kG + 8) / 2);
       }
     }
     if constexpr (!kDiag) {
