@@ -85,7 +85,7 @@ class _CsrEntry:
     checked with (seq_key; None: every row is valid)."""
 
     __slots__ = ("row_ptr", "col_idx", "sched", "n_slots", "stream", "window", "seq_key",
-                 "seq_ref", "pending", "sched_host", "sched_ready", "unchecked")
+                 "seq_ref", "pending", "sched_ready", "unchecked")
 
     def __init__(self, row_ptr, col_idx, sched, n_slots, stream, window, seq_key, seq_ref):
         self.row_ptr = weakref.ref(row_ptr)
@@ -99,7 +99,6 @@ class _CsrEntry:
         # Unchecked CSRs (USAGI_BSA_VALIDATE=0): (event, pinned row_ptr, pinned col_idx, B, H,
         # nqb) of the host copy still in flight, or None.
         self.pending = None
-        self.sched_host = None
         # Event after an asynchronous copy of the plan to the device (or None: the copy was
         # synchronous); a launch on another stream waits for it.
         self.sched_ready = None
@@ -293,9 +292,8 @@ def _plan_rows(e: _CsrEntry, rp, B, H, nqb, dev, generic: bool, pinned=False) ->
     if sched is None:
         return
     src = torch.from_numpy(sched)
-    if pinned:  # copied behind the stream's queued work, no synchronisation
-        src = src.pin_memory()
-        e.sched_host = src  # stays alive until the copy has run
+    if pinned:  # copied behind the stream's queued work, no synchronisation; torch keeps the pinned
+        src = src.pin_memory()  # memory from being reused until the copy has run
     e.sched = src.to(dev, non_blocking=pinned)
     e.n_slots = len(sched)
     e.stream = torch.cuda.current_stream(dev) if dev.type == "cuda" else None
