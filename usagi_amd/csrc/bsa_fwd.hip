@@ -910,16 +910,16 @@ LaunchEvents take_events() {
 //   n = 48,  T 1024, w 2:  dma 9.0 / 9.7   pipe 7.6 / 8.9   32: 6.6 / 6.8
 //   n = 64,  T 1024, w 8:  dma 18.6 / 22.4                  32: 9.5 / 10.5   64: 13.5 / 15.8
 //   n = 96,  T 1024, w 8:  dma 19.1 / 22.6                  32: 13.6 / 14.5  64: 13.9 / 16.0
-//   n = 128, T 4096, w 16: dma 32.2 / 40.2                  32: 26.2 / 30.3  64: 21.0 / 25.4
-//   n = 256, T 4096, w 16: dma 32.4 / 40.1                  64: 40.8 / 48.7  128: 30.5 / 34.8
+//   n = 128, T 4096, w 16: dma 32.2 / 40.2                  32: 26.2 / 30.3  64: 21.0 / 24.6
+//   n = 256, T 4096, w 16: dma 32.4 / 40.1                  64: 40.8 / 48.7  128: 30.5 / 32.5
 //   n = 256, T 1024, w 4:  dma 12.6 / 14.4                                   128: 13.1 / 14.5
 // so the line to 32 rows lies at 64 query blocks (256 workgroups, one per CU), to 64 rows at 128
-// and to 128 rows at 256, the last only for rows of 6 blocks and more. Rows that grow towards the end
-// of the sequence leave the chip emptier still: full causal rows of 32 blocks take 36 (64 rows)
-// against 52 (128) at n = 160 and 44 against 52 at n = 256, and where two workgroups of
-// bsa_fwd_dma_kernel share a CU until the longest row ends (n = 512: 89 / 102 us), 72 / 79 with 128
-// rows; with equal rows (w 8 at n = 512) it is 33 against 40, the other way round, and with rows of 16
-// blocks at most 49 against 54.
+// and to 128 rows at 256, the last only for rows of 6 blocks and more. Long rows that grow towards the
+// end of the sequence leave the chip emptier still: full causal rows of 32 blocks take 36 (64 rows)
+// against 52 (128) at n = 160 and 44 against 52 at n = 256 (of 8 blocks at n = 256: 24 against 18), and
+// where two workgroups of bsa_fwd_dma_kernel share a CU until the longest row ends (n = 512: 89 / 102
+// us), 71 / 75 with 128 rows; with equal rows (w 8 at n = 512) it is 33 against 40, the other way
+// round, and with full causal rows of 16 blocks 49 against 54.
 constexpr long long kPipeMaxBlocks = 4;
 constexpr int kSmall32 = 64;
 constexpr int kSmall64 = 128;
@@ -953,7 +953,7 @@ int small_query_rows(const Args& a, int kRows, long long entries) {
   const double longest = kRows == kRowsGeneric ? mean : causal_row(entries, a.nqb);
   if (a.n_items <= kSmall128) {
     if (longest < 6.0) return 0;
-    return longest >= 1.75 * mean ? 64 : 128;
+    return mean >= 12.0 && longest >= 1.75 * mean ? 64 : 128;
   }
   return mean >= 12.0 && longest >= 1.5 * mean ? 128 : 0;
 }

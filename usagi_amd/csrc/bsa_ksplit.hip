@@ -18,12 +18,12 @@
 //
 // What a row of 8 blocks takes (sliding window, fp16 / bf16, kernel time in us, one box):
 //   query blocks   bsa_fwd_dma_kernel   bsa_ksplit_kernel   bsa_wide_kernel<4>   <2>
-//   64             18.6 / 22.6          9.7 / 11.0          13.6 / 15.8          18.1 / 20.6
-//   128            18.9 / 22.9          17.9 / 20.6         13.8 / 16.0          18.4 / 20.7
-//   256            19.3 / 23.2          30.7 / 35.2         26.2 / 30.2          18.6 / 21.0
+//   64             18.6 / 22.6          9.5 / 10.5          13.6 / 15.5          18.1 / 19.8
+//   128            18.9 / 22.9          17.9 / 20.6         13.7 / 15.4          18.4 / 19.8
+//   256            19.3 / 23.2          30.7 / 35.2         26.2 / 29.5          18.6 / 20.0
 // Per block that is 0.5, 0.85 and 1.3 us against 1.75-2.3 us (one workgroup of bsa_fwd_dma_kernel on
-// a CU); what is left bounds is instruction issue: a step of bsa_wide_kernel<2> is 3,500 cycles, of
-// which a wave's MFMAs are 1,024, and its DMA wait 50.
+// a CU). What is left bounds is the chain of a step: Q·K^T, softmax and P·V of bsa_wide_kernel<2> take
+// 3,500 cycles for 1,024 cycles of a wave's MFMAs (2,048 of its SIMD's), its DMA wait 50 of them.
 #include "bsa_device.h"
 
 #include "bsa_internal.h"
