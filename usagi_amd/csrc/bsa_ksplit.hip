@@ -16,7 +16,7 @@
 // at the end of the row. One workgroup per CU (128 KiB of LDS): K and V are double-buffered and
 // requested a whole block (bsa_ksplit_kernel: two) ahead, so no DMA latency is exposed.
 //
-// What a row of 8 blocks takes (sliding window, fp16 / bf16, kernel time in us, one box):
+// What a row of 8 blocks takes (sliding window, fp16 / bf16, kernel time in us):
 //   query blocks   bsa_fwd_dma_kernel   bsa_ksplit_kernel   bsa_wide_kernel<4>   <2>
 //   64             18.6 / 22.6          9.5 / 10.5          13.6 / 15.5          18.1 / 19.8
 //   128            18.9 / 22.9          17.9 / 20.6         13.7 / 15.4          18.4 / 19.8
