@@ -20,7 +20,8 @@
  *     diagonal give the same result). The diagonal is processed implicitly and causally masked;
  *     entries before it are processed unmasked (kernels/v7_blockptr_warpspec.py:83-136).
  *   - seq_lens: int32 [B] or NULL (NULL: every sequence has length T). Query rows at or past
- *     seq_len get O = 0 and LSE = -inf (kernels/v7_blockptr_warpspec.py:63-67, 138-148).
+ *     seq_len get O = 0 and LSE = -inf (kernels/v7_blockptr_warpspec.py:63-67, 138-148). What q, k
+ *     and v hold there is not used: it may be NaN or infinite.
  *   - lse: float32 [B, H, T], natural-log log-sum-exp of the scaled scores, or NULL to skip.
  *   - sched / n_slots: an optional work plan from usagi_bsa_plan (device copy of its int32 array
  *     and its return value), or NULL / 0 for the kernel's built-in order. Any plan of the same

@@ -11,7 +11,8 @@ import torch
 
 from oracle import c_ref
 from tests._helpers import assert_close
-from usagi_amd import block_sparse_attn_fwd, block_sparse_attn_fwd_generic
+from usagi_amd import (block_sparse_attn_fwd, block_sparse_attn_fwd_generic,
+                       block_sparse_attn_fwd_window)
 from usagi_amd import patterns as P
 
 pytestmark = pytest.mark.gpu
@@ -112,6 +113,48 @@ def test_rows_past_seq_len_hold_anything(H, dtype):
     torch.cuda.synchronize()
     oo, ol = c_ref.fwd(q.float().numpy(), k.float().numpy(), v.float().numpy(), rp, ci,
                        np.asarray(sl, np.int32), round_p_fp16=False)
+    rtol = 2e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0)
+    assert_close(o.float().cpu().numpy(), oo, rtol=rtol)
+    assert_close(lse.cpu().numpy(), ol, what="LSE")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+# n = 32, 128, 256 and 640: 32, 64 and 128 query rows per workgroup, and bsa_fwd_dma_kernel
+@pytest.mark.parametrize("H", [2, 8, 16, 40])
+@pytest.mark.parametrize("entry", ["csr", "window", "generic"])
+@pytest.mark.parametrize("sl", [(609, 33), (1, 895)])
+def test_tail_inside_a_step_of_32_keys(sl, entry, H, dtype):
+    """q, k and v past seq_len are NaN or infinite and seq_len lies inside the 32 keys of a P·V step:
+    the rows before it are those of clean inputs. Generic rows list blocks that seq_len cuts above
+    the diagonal too."""
+    B, T, w = 2, 1024, 7
+    nqb = T // 128
+    if entry == "generic":
+        rng = np.random.default_rng(H)
+        rp, ci = P.make_csr(B, H, T, lambda b, h, i: [int(x) for x in rng.permutation(nqb)[:w]])
+    else:
+        rp, ci = P.sliding_csr(B, H, T, w)
+    q, k, v = P.make_qkv(B, H, T, seed=H, dtype=dtype)
+    dirty = [x.clone() for x in (q, k, v)]
+    for x, bad in zip(dirty, (float("nan"), float("nan"), float("inf"))):
+        for b in range(B):
+            x[b, :, sl[b]:] = bad
+            x[b, :, sl[b] + 1::2] = float("nan")
+    dirty = [x.to(DEV) for x in dirty]
+    drp, dci = torch.from_numpy(rp).to(DEV), torch.from_numpy(ci).to(DEV)
+    dsl = torch.tensor(sl, dtype=torch.int32, device=DEV)
+    print(f"case tail in a step {entry} H{H} {dtype} seq_lens={sl}", flush=True)
+    if entry == "window":
+        o, lse = block_sparse_attn_fwd_window(*dirty, w, 0, dsl)
+    elif entry == "generic":
+        o, lse = block_sparse_attn_fwd_generic(*dirty, drp, dci, dsl)
+    else:  # not routed to the analytic rows: two entries of one row in the other order
+        ci2 = ci.copy()
+        ci2[0, 0, rp[0, 0, 4]:rp[0, 0, 4] + 2] = ci[0, 0, rp[0, 0, 4]:rp[0, 0, 4] + 2][::-1]
+        o, lse = block_sparse_attn_fwd(*dirty, drp, torch.from_numpy(ci2).to(DEV), dsl)
+    torch.cuda.synchronize()
+    oo, ol = c_ref.fwd(q.float().numpy(), k.float().numpy(), v.float().numpy(), rp, ci,
+                       np.asarray(sl, np.int32), round_p_fp16=False, generic=entry == "generic")
     rtol = 2e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0)
     assert_close(o.float().cpu().numpy(), oo, rtol=rtol)
     assert_close(lse.cpu().numpy(), ol, what="LSE")

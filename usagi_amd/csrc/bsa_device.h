@@ -174,6 +174,18 @@ __device__ __forceinline__ uint32_t lds_addr_of(const void* p) {
   return (uint32_t)(uintptr_t)(lds_void*)p;
 }
 
+// Zeroes rows `from` and above of a wave's kSliceRows rows of V in LDS (256 bytes a row; from <= 0: all
+// of them). V past seq_len may hold anything, and P = 0 does not cancel a NaN or an infinity there. Runs
+// only on the key blocks that seq_len cuts. A row at a time and 4 bytes a lane, with the address made
+// here: wider stores, or an address made ahead of the branch, spill in the bf16 generic kernel.
+template <int kSliceRows>
+__device__ __forceinline__ void zero_v_tail(char* slice, int lane, int from) {
+  asm volatile("" : "+v"(lane));
+  uint32_t* row = (uint32_t*)slice + lane;
+#pragma unroll 1
+  for (int r = max(from, 0); r < kSliceRows; ++r) row[r * (kHd / 2)] = 0;
+}
+
 #define USAGI_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 #define USAGI_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
 #define USAGI_FENCE() __builtin_amdgcn_sched_barrier(0)

@@ -315,6 +315,12 @@ void bsa_fwd_dma_kernel(Args a) {
     USAGI_BARRIER();   // K(j) complete; every wave is done reading V of the previous block
     const int kb = kDiag ? qb : key_block(j);
     const char* vt_src = tile_v(kb);
+    if constexpr (kGeneric && !kFullSeq && !kDiag) {
+      if (__builtin_expect(kb * kBlk >= seq_len, 0)) {  // all its keys are past seq_len: nothing but the next K tile to do
+        if constexpr (kNext) dma_tile8(tile_k(key_block(j + 1)), k_off, k_dst);
+        return;
+      }
+    }
 
     // Matrix-core sections run at raised wave priority, so when both waves of a SIMD (one per
     // workgroup) can issue, the MFMA stream goes first and the other wave's exponentials fill
@@ -524,6 +530,11 @@ void bsa_fwd_dma_kernel(Args a) {
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) *(u32x4*)(slice + (4 * h + i) * 1024) = x[i];
+      }
+    }
+    if constexpr (!kFullSeq && (kDiag || kGeneric)) {
+      if ((kb + 1) * kBlk > seq_len) {
+        zero_v_tail<32>((char*)v_lds + wave * 8192, lane, seq_len - kb * kBlk - 32 * wave);
       }
     }
     USAGI_BARRIER();   // every wave is done reading K(j); V(j) is complete

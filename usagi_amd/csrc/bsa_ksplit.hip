@@ -426,7 +426,9 @@ void bsa_ksplit_kernel(Args a) {
   // Q, the column chunk and the first K and V slices have landed (a real s_waitcnt: the compiler
   // then knows that no load of its own is outstanding inside the loop).
   __builtin_amdgcn_s_waitcnt(0x0F70);
-  if (n_blk > 1) fetch(row.key_block(1), 1);
+  // Key blocks of the next two steps.
+  int kb_next[2] = {kGeneric && n_blk > 0 ? row.key_block(0) : 0, n_blk > 1 ? row.key_block(1) : 0};
+  if (n_blk > 1) fetch(kb_next[1], 1);
   if (n_blk > 0) k_read(0);
 
   // Step i, the operands of its K already in kop. Requests in flight, oldest first, eight each:
@@ -438,11 +440,29 @@ void bsa_ksplit_kernel(Args a) {
     const int stage = i & 1;
     const bool next = kMore || i + 1 < n_blk;
     const uint32_t dst = wave_dst + stage * 2 * kSlice;
-    const int kb = kDiag ? qb : (kGeneric ? row.key_block(i) : 0);
+    const int kb = kDiag ? qb : kb_next[0];
     const int kb2 = kMore ? row.key_block(i + 2) : 0;
+    kb_next[0] = kb_next[1];
+    kb_next[1] = kb2;
     const char* k2 = k_head + (size_t)kb2 * kTileBytes;
     const char* v2 = v_head + (size_t)kb2 * kTileBytes;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if constexpr (kGeneric && !kDiag) {
+      if (__builtin_expect(kb * kBlk >= seq_len, 0)) {  // all its keys are past seq_len: nothing but the requests to do
+        if constexpr (kMore) {
+          dma_tile8(k2, k_off, dst);
+          USAGI_WAIT_VM(24);  // V(i) has landed: its slice can be written again
+          dma_tile8(v2, v_off, dst + kSlice);
+          USAGI_WAIT_VM(24);  // K(i+1) has landed
+        } else if (next) {
+          USAGI_WAIT_VM(8);
+        } else {
+          USAGI_WAIT_VM(0);  // V(i) has landed: O takes its place
+        }
+        if (next) k_read(stage ^ 1);
+        return;
+      }
+    }
 
     floatx4 st[2][2];
 #pragma unroll
@@ -495,8 +515,27 @@ void bsa_ksplit_kernel(Args a) {
         vop[u] = __builtin_bit_cast(half8, x);
       }
     }
-    // On the diagonal a wave whose keys all lie above the rows is skipped (its P is zero, but V past
-    // seq_len may hold anything).
+    if constexpr (kDiag || kGeneric) {
+      // V past seq_len may hold anything, and P = 0 does not cancel a NaN or an infinity there.
+      const int n_keys = seq_len - kb * kBlk - 32 * wave;  // of this wave's 32
+      if (__builtin_expect(n_keys < 32, 0)) {
+        const int n = n_keys - 4 * g4;
+        uint32_t keep[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const int e = 16 * (w >> 1) + 2 * (w & 1);
+          keep[w] = (e < n ? 0xffffu : 0u) | (e + 1 < n ? 0xffff0000u : 0u);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          u32x4 x = __builtin_bit_cast(u32x4, vop[u]);
+#pragma unroll
+          for (int w = 0; w < 4; ++w) x[w] &= keep[w];
+          vop[u] = __builtin_bit_cast(half8, x);
+        }
+      }
+    }
+    // On the diagonal a wave whose keys all lie above the rows is skipped.
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (!kDiag || wave <= sub) {
@@ -613,19 +652,44 @@ void bsa_wide_kernel(Args a) {
     }
   }
 
+  int kb_next = kGeneric && n_blk > 0 ? row.key_block(0) : 0;  // key block of the next step
   // Step i: the tiles of step i + 1 (kMore) are requested during Q·K^T into the other stage, whose
   // readers all passed this step's barrier.
   auto step = [&](auto diag_tag, auto more_tag, int i) {
     constexpr bool kDiag = decltype(diag_tag)::value;
     constexpr bool kMore = decltype(more_tag)::value;
     const int stage = i & 1;
-    const int kb = kDiag ? qb : (kGeneric ? row.key_block(i) : 0);
+    const int kb = kDiag ? qb : kb_next;
     const int kb1 = kMore ? row.key_block(i + 1) : 0;
+    kb_next = kb1;
     const char* k1 = k_head + (size_t)kb1 * kTileBytes;
     const char* v1 = v_head + (size_t)kb1 * kTileBytes;
     const uint32_t dst = dst0 + (stage ^ 1) * 2 * kTileBytes;
     USAGI_WAIT_VM(0);  // this wave's rows of K(i) and V(i) have landed (bf16: V(i) is in LDS as fp16)
+    if constexpr (kDiag || kGeneric) {
+      if (__builtin_expect((kb + 1) * kBlk > seq_len, 0)) {
+        char* rows = lds + (2 * stage + 1) * kTileBytes + wave * 4096;
+        const int n = seq_len - kb * kBlk - 16 * wave;
+        // V past seq_len may hold anything, and P = 0 does not cancel a NaN or an infinity there.
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          if (r + g4 >= n) *(u32x4*)(rows + r * 256 + lane * 16) = u32x4{0, 0, 0, 0};
+        }
+      }
+    }
     USAGI_BARRIER();
+    if constexpr (kGeneric && !kDiag) {
+      if (__builtin_expect(kb * kBlk >= seq_len, 0)) {  // all its keys are past seq_len: nothing but the next tiles to do
+        if constexpr (kMore) {
+          fetch(kb1, stage ^ 1);
+          if constexpr (kBf16) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) put_v(stage ^ 1, n);
+          }
+        }
+        return;
+      }
+    }
 
     // ---- S^T = K · Q^T: fragment f = kNT * ks + t, read four ahead.
     const char* k_rd = k_rd0 + stage * 2 * kTileBytes;
@@ -687,7 +751,7 @@ void bsa_wide_kernel(Args a) {
     softmax<kNT, kDiag>(st, s, scale, pb);
 
     // ---- O^T += V^T · P^T, fragment g = 8ks + u read four ahead. On the diagonal the 32-key steps
-    // above the wave's rows are skipped (their P is zero, but V past seq_len may hold anything).
+    // above the wave's rows are skipped.
     __builtin_amdgcn_s_setprio(1);
     auto v_read = [&](int g) { return v_fragment(v_rd + (g >> 3) * 8192 + 16 * ((2 * (g & 7)) ^ v_x)); };
     constexpr int kG = 8 * kKS;
