@@ -245,12 +245,11 @@ def _check_on_host(e: _CsrEntry, row_ptr, col_idx, B, H, nqb, dev, generic: bool
     _plan_entry(e, rp, ci, B, H, nqb, dev, generic)
 
 
-def _start_check(rp, ci, B, H, nqb, max_nnz, stream) -> tuple:
-    """Launch the GPU check of int32 device tensors; the forward launch follows it on the stream."""
-    cap = _native.check_cap(B * H * nqb)
-    result = torch.empty(cap, dtype=torch.int32, pin_memory=True)
+def _start_check(result, rp, ci, B, H, nqb, max_nnz, stream) -> tuple:
+    """Launch the GPU check of int32 device tensors; the forward launch follows it on the stream.
+    result: pinned memory that the caller keeps until the check has run."""
     n_flags = _native.check_csr_gpu(rp.data_ptr(), ci.data_ptr(), B, H, nqb, max_nnz,
-                                    result.data_ptr(), cap, stream)
+                                    result.data_ptr(), result.numel(), stream)
     done = torch.cuda.Event()
     done.record()
     return done, result, n_flags
@@ -410,18 +409,31 @@ def _run_csr(q, k, v, row_ptr, col_idx, seq_lens, generic: bool):
             if plan.sched_ready is not None:
                 current.wait_event(plan.sched_ready)
             plan.sched.record_stream(current)
-        check = _start_check(rp, ci, B, H, nqb, max_nnz, stream) if plan.unchecked is not None else None
-        _native.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), rp.data_ptr(),
-                    ci.data_ptr() if max_nnz else None, sl.data_ptr() if sl is not None else None,
-                    out.data_ptr(), lse.data_ptr(), B, H, T, D, max_nnz, _DTYPE_CODES[q.dtype],
-                    plan.sched.data_ptr() if plan.sched is not None else None, plan.n_slots,
-                    stream, generic=generic)
-        if check is not None:
+
+        def launch():
+            _native.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), rp.data_ptr(),
+                        ci.data_ptr() if max_nnz else None, sl.data_ptr() if sl is not None else None,
+                        out.data_ptr(), lse.data_ptr(), B, H, T, D, max_nnz, _DTYPE_CODES[q.dtype],
+                        plan.sched.data_ptr() if plan.sched is not None else None, plan.n_slots,
+                        stream, generic=generic)
+
+        if plan.unchecked is None:
+            launch()
+            return out, lse
+        result = torch.empty(_native.check_cap(B * H * nqb), dtype=torch.int32, pin_memory=True)
+        try:
+            check = _start_check(result, rp, ci, B, H, nqb, max_nnz, stream)
+            launch()
             entries = _finish_check(plan, check, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
-            if plan.window is not None and entries != max_nnz:
-                # A padded column list may have led to another kernel than the later calls' analytic
-                # rows, whose results differ in the last bits: this call gives theirs.
-                launch_window()
+        except BaseException:
+            # The check may be queued still, and torch does not know that it writes to the result:
+            # the memory must not go back before it has run.
+            torch.cuda.current_stream(dev).synchronize()
+            raise
+        if plan.window is not None and entries != max_nnz:
+            # A padded column list may have led to another kernel than the later calls' analytic
+            # rows, whose results differ in the last bits: this call gives theirs.
+            launch_window()
     return out, lse
 
 
