@@ -28,7 +28,7 @@
  *     CSR gives bit-identical results: it only decides which GPU slot runs which query block.
  *   - stream: a hipStream_t (NULL = the default stream). The launch is asynchronous.
  *   - Kernel: chosen per call from the number of query blocks n = B*H*T/128 and the entries per
- *     head (max_nnz, or the analytic pattern's own count). Few query blocks (n <= 128, n <= 256 with
+ *     head (max_nnz, the analytic pattern's own count, or what usagi_bsa_fwd_entries is told). Few query blocks (n <= 128, n <= 256 with
  *     rows of 6 blocks and more, n <= 512 with long rows that grow as full causal ones do) run
  *     kernels that divide the keys of a block over the waves. Other calls without seq_lens whose
  *     rows hold at most 4 key blocks on average (already from n = 64 on) run a software-pipelined
@@ -89,6 +89,26 @@ int usagi_bsa_fwd_generic(const void* q, const void* k, const void* v,
                           int32_t batch, int32_t heads, int32_t seq_len, int32_t head_dim,
                           int32_t max_nnz, int32_t dtype, const int32_t* sched,
                           int32_t n_slots, void* stream);
+
+/* usagi_bsa_fwd (generic = 0) or usagi_bsa_fwd_generic (generic != 0) for a CSR whose entries are known:
+ * `entries` are those of the head that holds most of them (the largest last value of row_ptr), < 0 if
+ * unknown. The kernel is then chosen by them where col_idx is wider than its rows need. Same arguments
+ * otherwise. */
+int usagi_bsa_fwd_entries(const void* q, const void* k, const void* v,
+                          const int32_t* row_ptr, const int32_t* col_idx,
+                          const int32_t* seq_lens, void* out, float* lse,
+                          int32_t batch, int32_t heads, int32_t seq_len, int32_t head_dim,
+                          int32_t max_nnz, int32_t dtype, const int32_t* sched,
+                          int32_t n_slots, void* stream, int32_t generic, int32_t entries);
+
+/* The kernel such a call runs: two calls of which it returns the same run the same kernel (whose results
+ * on one CSR are bit-identical). USAGI_BSA_KERNEL_TWO_PHASE, USAGI_BSA_KERNEL_PIPELINED, or the query rows
+ * per workgroup (32, 64, 128) of a kernel for few query blocks; negative: a rejected size. Analytic rows
+ * run the kernel of a CSR with max_nnz = their entries per head. */
+#define USAGI_BSA_KERNEL_TWO_PHASE 0
+#define USAGI_BSA_KERNEL_PIPELINED 1
+int usagi_bsa_kernel_of(int32_t batch, int32_t heads, int32_t seq_len, int32_t with_seq_lens,
+                        int32_t max_nnz, int32_t generic, int32_t entries);
 
 /* Forward pass over an analytic pattern instead of a CSR: query block qb attends the global
  * prefix 0 .. n_global-1 and the window max(0, qb-window+1) .. qb (deduplicated; the diagonal is

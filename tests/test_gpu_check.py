@@ -124,3 +124,48 @@ def test_first_call_equals_later_calls(pad):
     with pytest.raises(ValueError, match="h=3"):
         block_sparse_attn_fwd(*dev, None)
     submission.clear_csr_cache()
+
+
+@pytest.mark.parametrize("H,T,width", [(8, 4096, 528), (16, 4096, 528), (4, 8192, 2080), (3, 5504, 946),
+                                       (8, 8320, 4225)])
+def test_padded_list_equals_the_list_of_its_rows(H, T, width, monkeypatch):
+    """A column list allocated for full causal rows or more: every call, the first one too, gives the
+    bits of the list that just holds the rows (so runs the same kernel), and only a first call whose
+    width led to another kernel launches twice."""
+    submission.clear_csr_cache()
+    rp, ci = P.retrieval_csr(1, H, T, 6, 3)
+    wide = np.concatenate([ci, np.zeros((1, H, width - ci.shape[-1]), np.int32)], axis=-1)
+    qkv = [x.cuda() for x in P.make_qkv(1, H, T, seed=H)]
+    drp, dci, dwide = (torch.from_numpy(x).cuda() for x in (rp, ci, wide))
+    launches = []
+    fwd = _native.fwd
+    monkeypatch.setattr(_native, "fwd", lambda *a, **kw: (launches.append(1), fwd(*a, **kw)))
+    print(f"case padded list H{H} T{T} width {width}", flush=True)
+    o, l = block_sparse_attn_fwd(*qkv, drp, dci, None)
+    for call in range(2):
+        launches.clear()
+        ow, lw = block_sparse_attn_fwd(*qkv, drp, dwide, None)
+        torch.cuda.synchronize()
+        assert torch.equal(o, ow) and torch.equal(l, lw)
+        twice = _native.kernel_of(1, H, T, False, width) != _native.kernel_of(1, H, T, False, ci.shape[-1])
+        assert len(launches) == (2 if twice and call == 0 else 1)
+    submission.clear_csr_cache()
+
+
+def test_padded_window_of_the_same_kernel_launches_once(monkeypatch):
+    submission.clear_csr_cache()
+    B, H, T = 1, 8, 8320
+    rp, ci = P.sliding_csr(B, H, T, 8)
+    ci = np.concatenate([ci, np.zeros((B, H, 900), np.int32)], axis=-1)
+    dev = [x.cuda() for x in P.make_qkv(B, H, T, seed=5)] + [torch.from_numpy(x).cuda() for x in (rp, ci)]
+    launches = []
+    for name in ("fwd", "fwd_window"):
+        f = getattr(_native, name)
+        monkeypatch.setattr(_native, name, lambda *a, f=f, **kw: (launches.append(1), f(*a, **kw)))
+    print("case padded window, one launch", flush=True)
+    o1, l1 = block_sparse_attn_fwd(*dev, None)
+    assert len(launches) == 1
+    o2, l2 = block_sparse_attn_fwd(*dev, None)
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2) and torch.equal(l1, l2)
+    submission.clear_csr_cache()

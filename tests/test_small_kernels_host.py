@@ -1,4 +1,4 @@
-"""CPU checks of bsa_ksplit.hip and bsa_check.hip: the gfx950 assembly spills nothing, emits no
+"""CPU checks of the choice among the kernels and of bsa_ksplit.hip and bsa_check.hip: the gfx950 assembly spills nothing, emits no
 packed-FP32 instruction and writes M0 only right before an LDS DMA; the GPU check's entry point rejects
 bad arguments before any launch."""
 
@@ -56,3 +56,25 @@ def test_gpu_check_rejects_bad_arguments(over):
     code = _native.load().usagi_bsa_check_csr_gpu(a["rp"], a["ci"], a["B"], a["H"], a["nqb"], a["nnz"],
                                                   a["result"], a["cap"], a["stream"])
     assert code < 0 and _native.last_error()
+
+
+@pytest.mark.parametrize("with_seq_lens", [False, True])
+@pytest.mark.parametrize("H,nqb", [(3, 43), (8, 32), (10, 32), (16, 32), (4, 64), (8, 64), (33, 16)])
+@pytest.mark.parametrize("w", [5, 8, 16])
+def test_a_padded_column_list_runs_the_kernel_of_its_rows(w, H, nqb, with_seq_lens):
+    """Once the entries are known, the width of col_idx does not decide between the kernels for few
+    query blocks and bsa_fwd_dma_kernel."""
+    nnz = sum(min(i + 1, w) for i in range(nqb))
+    want = _native.kernel_of(1, H, nqb * 128, with_seq_lens, nnz)
+    for width in (nnz + 1, nqb * (nqb + 1) // 2, nqb * nqb):
+        assert _native.kernel_of(1, H, nqb * 128, with_seq_lens, max(width, nnz), False, nnz) == want
+    # more entries than the list is wide count as its width
+    assert _native.kernel_of(1, H, nqb * 128, with_seq_lens, nnz, False, nqb * nqb) == want
+
+
+def test_kernel_of_and_fwd_entries_reject_what_the_forward_rejects():
+    lib = _native.load()
+    for B, H, T, nnz in ((0, 1, 128, 1), (1, 0, 128, 1), (1, 1, 100, 1), (1, 1, 128, -1), (64, 64, 1 << 20, 1)):
+        assert lib.usagi_bsa_kernel_of(B, H, T, 0, nnz, 0, -1) < 0 and _native.last_error()
+        assert lib.usagi_bsa_fwd_entries(1, 1, 1, 1, 1, None, 1, None, B, H, T, 128, nnz, 0, None, 0, None,
+                                         0, 1) < 0

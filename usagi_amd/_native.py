@@ -19,6 +19,8 @@ BF16 = 1
 EXPORTED_SYMBOLS = (
     "usagi_bsa_fwd",
     "usagi_bsa_fwd_generic",
+    "usagi_bsa_fwd_entries",
+    "usagi_bsa_kernel_of",
     "usagi_bsa_fwd_window",
     "usagi_bsa_check_csr",
     "usagi_bsa_check_csr_gpu",
@@ -55,6 +57,10 @@ def load() -> ctypes.CDLL:
     lib.usagi_bsa_fwd.restype = ctypes.c_int
     lib.usagi_bsa_fwd_generic.argtypes = fwd_args
     lib.usagi_bsa_fwd_generic.restype = ctypes.c_int
+    lib.usagi_bsa_fwd_entries.argtypes = fwd_args + [i32, i32]
+    lib.usagi_bsa_fwd_entries.restype = ctypes.c_int
+    lib.usagi_bsa_kernel_of.argtypes = [i32] * 7
+    lib.usagi_bsa_kernel_of.restype = ctypes.c_int
     lib.usagi_bsa_fwd_window.argtypes = [p, p, p, i32, i32, p, p, p, i32, i32, i32, i32, i32, p]
     lib.usagi_bsa_fwd_window.restype = ctypes.c_int
     lib.usagi_bsa_check_csr.argtypes = [p, p, p, i32, i32, i32, i32]
@@ -88,11 +94,27 @@ def check(code: int) -> None:
 
 def fwd(q_ptr, k_ptr, v_ptr, row_ptr_ptr, col_idx_ptr, seq_lens_ptr, out_ptr, lse_ptr,
         batch, heads, seq_len, head_dim, max_nnz, dtype, sched_ptr, n_slots, stream,
-        generic: bool = False) -> None:
+        generic: bool = False, entries: int = -1) -> None:
     lib = load()
+    if 0 <= entries < max_nnz:
+        check(lib.usagi_bsa_fwd_entries(q_ptr, k_ptr, v_ptr, row_ptr_ptr, col_idx_ptr, seq_lens_ptr,
+                                        out_ptr, lse_ptr, batch, heads, seq_len, head_dim, max_nnz,
+                                        dtype, sched_ptr, n_slots, stream, 1 if generic else 0,
+                                        entries))
+        return
     f = lib.usagi_bsa_fwd_generic if generic else lib.usagi_bsa_fwd
     check(f(q_ptr, k_ptr, v_ptr, row_ptr_ptr, col_idx_ptr, seq_lens_ptr, out_ptr, lse_ptr, batch,
             heads, seq_len, head_dim, max_nnz, dtype, sched_ptr, n_slots, stream))
+
+
+def kernel_of(batch, heads, seq_len, with_seq_lens: bool, max_nnz, generic: bool = False,
+              entries: int = -1) -> int:
+    """Which kernel a CSR call runs (usagi_bsa_kernel_of)."""
+    code = load().usagi_bsa_kernel_of(batch, heads, seq_len, 1 if with_seq_lens else 0, max_nnz,
+                                      1 if generic else 0, entries)
+    if code < 0:
+        raise NativeError(code, last_error())
+    return code
 
 
 def fwd_window(q_ptr, k_ptr, v_ptr, window, n_global, seq_lens_ptr, out_ptr, lse_ptr,

@@ -974,7 +974,12 @@ struct Choice {
   int query_rows;  // bsa_ksplit.hip kernel, or 0
 };
 
-Choice choose(const Args& a, int kRows) {
+// known: entries of the head that holds most of them, or -1 where only the width of the column list is
+// known. The few-query-block rules go by it: a list allocated for full causal rows and holding rows of 8
+// blocks took 27 us instead of 20 at n = 256 and 40 instead of 33 at n = 512 (T 4096) as full causal rows.
+// The short-row rule goes by the width alone: with it known that the rows of such a list are short,
+// bsa_fwd_dma_kernel is the faster one (w 2, n = 512, T 4096: 14 us against 17).
+Choice choose(const Args& a, int kRows, int known) {
   const long long entries = row_entries(a, kRows);
   if (kRows != kRowsGeneric && !a.seq_lens) {
     const char* e = getenv("USAGI_BSA_PIPE");
@@ -982,15 +987,15 @@ Choice choose(const Args& a, int kRows) {
     // From 64 query blocks on short rows keep the pipelined kernel.
     if (!(e && e[0] == '0') && entries <= kPipeMaxBlocks * a.nqb && a.n_items >= kSmall32) return {true, 0};
   }
-  return {false, small_query_rows(a, kRows, entries)};
+  return {false, small_query_rows(a, kRows, known >= 0 && known < entries ? known : entries)};
 }
 
 template <bool kBf16, int kRows>
-int launch(const Args& a, hipStream_t s, LaunchEvents ev) {
+int launch(const Args& a, int known, hipStream_t s, LaunchEvents ev) {
   const void* fn = a.seq_lens
                        ? reinterpret_cast<const void*>(&bsa_fwd_dma_kernel<kBf16, kRows, false>)
                        : reinterpret_cast<const void*>(&bsa_fwd_dma_kernel<kBf16, kRows, true>);
-  const Choice c = choose(a, kRows);
+  const Choice c = choose(a, kRows, known);
   if constexpr (kRows == kRowsCsr || kRows == kRowsWindow) {
     if (c.pipe) fn = reinterpret_cast<const void*>(&bsa_fwd_pipe_kernel<kRows, kBf16>);
   }
@@ -1018,10 +1023,24 @@ int launch(const Args& a, hipStream_t s, LaunchEvents ev) {
 }
 
 template <int kRows>
-int launch_dtype(const Args& a, int32_t dtype, void* stream, LaunchEvents ev) {
+int launch_dtype(const Args& a, int known, int32_t dtype, void* stream, LaunchEvents ev) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == USAGI_BSA_BF16 ? launch<true, kRows>(a, s, ev)
-                                 : launch<false, kRows>(a, s, ev);
+  return dtype == USAGI_BSA_BF16 ? launch<true, kRows>(a, known, s, ev)
+                                 : launch<false, kRows>(a, known, s, ev);
+}
+
+int fwd_csr(int kRows, int known, const void* q, const void* k, const void* v, const int32_t* row_ptr,
+            const int32_t* col_idx, const int32_t* seq_lens, void* out, float* lse, int32_t batch,
+            int32_t heads, int32_t seq_len, int32_t head_dim, int32_t max_nnz, int32_t dtype,
+            const int32_t* sched, int32_t n_slots, void* stream) {
+  usagi_bsa_clear_error();
+  const LaunchEvents ev = take_events();
+  Args a;
+  int rc = prepare(a, q, k, v, seq_lens, out, lse, batch, heads, seq_len, head_dim, dtype);
+  if (rc == USAGI_BSA_OK) rc = prepare_csr(a, row_ptr, col_idx, max_nnz, sched, n_slots);
+  if (rc != USAGI_BSA_OK) return rc;
+  return kRows == kRowsGeneric ? launch_dtype<kRowsGeneric>(a, known, dtype, stream, ev)
+                               : launch_dtype<kRowsCsr>(a, known, dtype, stream, ev);
 }
 
 }  // namespace
@@ -1039,13 +1058,8 @@ extern "C" int usagi_bsa_fwd(const void* q, const void* k, const void* v,
                              int32_t heads, int32_t seq_len, int32_t head_dim, int32_t max_nnz,
                              int32_t dtype, const int32_t* sched, int32_t n_slots,
                              void* stream) {
-  usagi_bsa_clear_error();
-  const LaunchEvents ev = take_events();
-  Args a;
-  int rc = prepare(a, q, k, v, seq_lens, out, lse, batch, heads, seq_len, head_dim, dtype);
-  if (rc == USAGI_BSA_OK) rc = prepare_csr(a, row_ptr, col_idx, max_nnz, sched, n_slots);
-  if (rc != USAGI_BSA_OK) return rc;
-  return launch_dtype<kRowsCsr>(a, dtype, stream, ev);
+  return fwd_csr(kRowsCsr, -1, q, k, v, row_ptr, col_idx, seq_lens, out, lse, batch, heads, seq_len, head_dim,
+                 max_nnz, dtype, sched, n_slots, stream);
 }
 
 extern "C" int usagi_bsa_fwd_generic(const void* q, const void* k, const void* v,
@@ -1054,13 +1068,32 @@ extern "C" int usagi_bsa_fwd_generic(const void* q, const void* k, const void* v
                                      int32_t batch, int32_t heads, int32_t seq_len,
                                      int32_t head_dim, int32_t max_nnz, int32_t dtype,
                                      const int32_t* sched, int32_t n_slots, void* stream) {
+  return fwd_csr(kRowsGeneric, -1, q, k, v, row_ptr, col_idx, seq_lens, out, lse, batch, heads, seq_len, head_dim,
+                 max_nnz, dtype, sched, n_slots, stream);
+}
+
+extern "C" int usagi_bsa_fwd_entries(const void* q, const void* k, const void* v,
+                                     const int32_t* row_ptr, const int32_t* col_idx,
+                                     const int32_t* seq_lens, void* out, float* lse,
+                                     int32_t batch, int32_t heads, int32_t seq_len,
+                                     int32_t head_dim, int32_t max_nnz, int32_t dtype,
+                                     const int32_t* sched, int32_t n_slots, void* stream,
+                                     int32_t generic, int32_t entries) {
+  return fwd_csr(generic ? kRowsGeneric : kRowsCsr, entries, q, k, v, row_ptr, col_idx, seq_lens, out,
+                 lse, batch, heads, seq_len, head_dim, max_nnz, dtype, sched, n_slots, stream);
+}
+
+extern "C" int usagi_bsa_kernel_of(int32_t batch, int32_t heads, int32_t seq_len, int32_t with_seq_lens,
+                                   int32_t max_nnz, int32_t generic, int32_t entries) {
+  static const int32_t some = 0;  // stands for tensors that are there; not read
   usagi_bsa_clear_error();
-  const LaunchEvents ev = take_events();
   Args a;
-  int rc = prepare(a, q, k, v, seq_lens, out, lse, batch, heads, seq_len, head_dim, dtype);
-  if (rc == USAGI_BSA_OK) rc = prepare_csr(a, row_ptr, col_idx, max_nnz, sched, n_slots);
+  int rc = prepare(a, &some, &some, &some, with_seq_lens ? &some : nullptr, const_cast<int32_t*>(&some),
+                   nullptr, batch, heads, seq_len, kHd, USAGI_BSA_FP16);
+  if (rc == USAGI_BSA_OK) rc = prepare_csr(a, &some, &some, max_nnz, nullptr, 0);
   if (rc != USAGI_BSA_OK) return rc;
-  return launch_dtype<kRowsGeneric>(a, dtype, stream, ev);
+  const Choice c = choose(a, generic ? kRowsGeneric : kRowsCsr, entries);
+  return c.pipe ? USAGI_BSA_KERNEL_PIPELINED : c.query_rows;
 }
 
 extern "C" int usagi_bsa_fwd_window(const void* q, const void* k, const void* v,
@@ -1077,5 +1110,5 @@ extern "C" int usagi_bsa_fwd_window(const void* q, const void* k, const void* v,
   if (n_global < 0) return usagi_bsa_fail(USAGI_BSA_EINVAL, "n_global must be >= 0, got %d", (int)n_global);
   a.window = window;
   a.n_global = n_global;
-  return launch_dtype<kRowsWindow>(a, dtype, stream, ev);
+  return launch_dtype<kRowsWindow>(a, -1, dtype, stream, ev);
 }

@@ -73,6 +73,8 @@ _raw_stream = torch._C._cuda_getCurrentRawStream
 
 _NOTHING = contextlib.nullcontext()
 
+_INT32_MAX = 2 ** 31 - 1
+
 # Query blocks up to which no work plan is made: they all run at once (one workgroup per CU or more).
 _PLAN_ITEMS = 256
 
@@ -85,7 +87,7 @@ class _CsrEntry:
     checked with (seq_key; None: every row is valid)."""
 
     __slots__ = ("row_ptr", "col_idx", "sched", "n_slots", "stream", "window", "seq_key",
-                 "seq_ref", "pending", "sched_ready", "unchecked")
+                 "seq_ref", "pending", "sched_ready", "unchecked", "entries")
 
     def __init__(self, row_ptr, col_idx, sched, n_slots, stream, window, seq_key, seq_ref):
         self.row_ptr = weakref.ref(row_ptr)
@@ -102,6 +104,9 @@ class _CsrEntry:
         # Event after an asynchronous copy of the plan to the device (or None: the copy was
         # synchronous); a launch on another stream waits for it.
         self.sched_ready = None
+        # Entries of the head that holds most of them, or -1 (not known): the width of the column list
+        # may be far above.
+        self.entries = -1
         # The key of an entry that is not in the cache yet (else None): the call that made it checks
         # the CSR on the GPU (_start_check, _finish_check) around its launch.
         self.unchecked = None
@@ -256,11 +261,10 @@ def _start_check(result, rp, ci, B, H, nqb, max_nnz, stream) -> tuple:
 
 
 def _finish_check(e: _CsrEntry, check: tuple, row_ptr, col_idx, B, H, nqb, dev, generic: bool,
-                  seq_lens) -> int:
+                  seq_lens) -> None:
     """Wait for the check (the forward kernel is queued behind it or running), keep what it found in
     the entry and the entry in the cache; a CSR that it rejects is looked at again on the host, which
-    raises with the row's position or accepts the rows before seq_len. Returns the entries of the
-    first head."""
+    raises with the row's position or accepts the rows before seq_len."""
     import numpy as np
 
     done, result, n_flags = check
@@ -272,14 +276,15 @@ def _finish_check(e: _CsrEntry, check: tuple, row_ptr, col_idx, B, H, nqb, dev, 
         _check_on_host(e, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
     else:
         rows = B * H * nqb
+        lengths = r[n_flags + 2:n_flags + 2 + rows].reshape(B * H, nqb)
+        e.entries = min(int(lengths.sum(axis=1, dtype=np.int64).max()), _INT32_MAX)
         if rows > _PLAN_ITEMS:
             rp = np.zeros((B * H, nqb + 1), dtype=np.int32)
-            np.cumsum(r[n_flags + 2:n_flags + 2 + rows].reshape(B * H, nqb), axis=1, out=rp[:, 1:])
+            np.cumsum(lengths, axis=1, out=rp[:, 1:])
             _plan_rows(e, rp, B, H, nqb, dev, generic, pinned=True)
         if not generic and ROUTE_WINDOW and not flags & 2 and e.sched is None:
             e.window = (int(r[n_flags]), int(r[n_flags + 1]))
     _remember(e, key)
-    return int(r[n_flags + 2:n_flags + 2 + nqb].sum())
 
 
 def _plan_rows(e: _CsrEntry, rp, B, H, nqb, dev, generic: bool, pinned=False) -> None:
@@ -302,7 +307,8 @@ def _plan_rows(e: _CsrEntry, rp, B, H, nqb, dev, generic: bool, pinned=False) ->
 
 
 def _plan_entry(e: _CsrEntry, rp, ci, B, H, nqb, dev, generic: bool, pinned=False) -> None:
-    """Work plan and window pattern of a host copy of the CSR, into the entry."""
+    """Entries, work plan and window pattern of a host copy of the CSR, into the entry."""
+    e.entries = max(int(rp.max()), 0)
     _plan_rows(e, rp, B, H, nqb, dev, generic, pinned)
     if e.sched is None and not generic and ROUTE_WINDOW and ci.shape[-1]:
         e.window = window_pattern(rp, ci, nqb)
@@ -410,30 +416,37 @@ def _run_csr(q, k, v, row_ptr, col_idx, seq_lens, generic: bool):
                 current.wait_event(plan.sched_ready)
             plan.sched.record_stream(current)
 
-        def launch():
+        def launch(entries):
             _native.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), rp.data_ptr(),
                         ci.data_ptr() if max_nnz else None, sl.data_ptr() if sl is not None else None,
                         out.data_ptr(), lse.data_ptr(), B, H, T, D, max_nnz, _DTYPE_CODES[q.dtype],
                         plan.sched.data_ptr() if plan.sched is not None else None, plan.n_slots,
-                        stream, generic=generic)
+                        stream, generic=generic, entries=entries)
 
         if plan.unchecked is None:
-            launch()
+            launch(plan.entries)
             return out, lse
         result = torch.empty(_native.check_cap(B * H * nqb), dtype=torch.int32, pin_memory=True)
         try:
             check = _start_check(result, rp, ci, B, H, nqb, max_nnz, stream)
-            launch()
-            entries = _finish_check(plan, check, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
+            launch(-1)
+            _finish_check(plan, check, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
         except BaseException:
             # The check may be queued still, and torch does not know that it writes to the result:
             # the memory must not go back before it has run.
             torch.cuda.current_stream(dev).synchronize()
             raise
-        if plan.window is not None and entries != max_nnz:
-            # A padded column list may have led to another kernel than the later calls' analytic
-            # rows, whose results differ in the last bits: this call gives theirs.
-            launch_window()
+        if 0 <= plan.entries < max_nnz:
+            # A column list wider than its rows need may have led to another kernel than the later
+            # calls', whose results differ in the last bits: this call gives theirs.
+            lens = sl is not None
+            later = plan.entries if plan.window is not None else max_nnz
+            if (_native.kernel_of(B, H, T, lens, max_nnz, generic)
+                    != _native.kernel_of(B, H, T, lens, later, generic, plan.entries)):
+                if plan.window is not None:
+                    launch_window()
+                else:
+                    launch(plan.entries)
     return out, lse
 
 
