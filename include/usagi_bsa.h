@@ -149,6 +149,17 @@ int usagi_bsa_check_csr_gpu(const int32_t* row_ptr, const int32_t* col_idx, int3
                             int32_t heads, int32_t num_q_blocks, int32_t max_nnz, int32_t* result,
                             int32_t result_cap, void* stream);
 
+/* The same with seq_lens (DEVICE int32 [B], or NULL): bit 0 then says that a row before seq_len breaks a
+ * precondition, and bit 2 that a row of a query block at or past seq_len does, which a forward with these
+ * seq_lens never reads; such a row without entries in the list counts 0 entries. The flag words shifted
+ * right by USAGI_BSA_CHECK_FLAG_BITS hold row ends: the largest of them is the entries of the head that
+ * has most (usagi_bsa_fwd_entries). */
+#define USAGI_BSA_CHECK_FLAG_BITS 4
+int usagi_bsa_check_csr_gpu_lens(const int32_t* row_ptr, const int32_t* col_idx,
+                                 const int32_t* seq_lens, int32_t batch, int32_t heads,
+                                 int32_t num_q_blocks, int32_t max_nnz, int32_t* result,
+                                 int32_t result_cap, void* stream);
+
 /* Work plan over a HOST copy of row_ptr; no counterpart in the reference, whose grid is
  * (nqb, B*H) in index order (kernels/v7_blockptr_warpspec.py:178-179). When rows of different
  * heads differ in length, it spreads the work evenly over the GPU's 8 XCDs (each XCD on a few

@@ -169,3 +169,72 @@ def test_padded_window_of_the_same_kernel_launches_once(monkeypatch):
     torch.cuda.synchronize()
     assert torch.equal(o1, o2) and torch.equal(l1, l2)
     submission.clear_csr_cache()
+
+
+@pytest.mark.parametrize("how", ["none", "not diagonal", "above", "twice", "empty", "past the list"])
+@pytest.mark.parametrize("lens", [(2048, 2048), (2000, 1), (640, 641), (0, 129)])
+def test_rows_past_seq_len_against_the_host_check(lens, how):
+    """One broken row, before and past seq_len, in each of the sequences: the flags are the host
+    check's with and without seq_lens."""
+    B, H, T = 2, 3, 2048
+    nqb = T // 128
+    rng = np.random.default_rng(7)
+    sl = np.asarray(lens, np.int32)
+    dsl = torch.from_numpy(sl).cuda()
+    print(f"case check lens {lens} {how}", flush=True)
+    for _ in range(6):
+        rp, ci = P.retrieval_csr(B, H, T, 5, int(rng.integers(1 << 20)))
+        if how != "none":
+            broken(rp, ci, how, rng)
+
+        def rejected(seq_lens):
+            try:
+                _native.check_csr_host(rp, ci, B, H, nqb, ci.shape[-1], seq_lens=seq_lens)
+            except ValueError:
+                return True
+            return False
+
+        result = torch.empty(_native.check_cap(B * H * nqb), dtype=torch.int32, pin_memory=True)
+        drp, dci = torch.from_numpy(rp).cuda(), torch.from_numpy(ci).cuda()
+        n = _native.check_csr_gpu(drp.data_ptr(), dci.data_ptr(), B, H, nqb, ci.shape[-1],
+                                  result.data_ptr(), result.numel(),
+                                  torch.cuda.current_stream().cuda_stream, dsl.data_ptr())
+        torch.cuda.synchronize()
+        flags = int(np.bitwise_or.reduce(result.numpy()[:n]))
+        if how in ("none", "not diagonal", "above", "twice"):
+            assert int(result.numpy()[:n].max()) >> _native.CHECK_FLAG_BITS == rp[..., -1].max()
+        assert bool(flags & 1) == rejected(sl)
+        assert bool(flags & 5) == rejected(None)
+
+
+@pytest.mark.parametrize("on_host", [False, True])
+def test_rows_that_end_at_seq_len_are_checked_on_the_gpu(on_host, monkeypatch):
+    """A CSR without rows past seq_len, as a selector over ragged sequences makes it: no copy to the
+    host, one check for these seq_lens, another for other ones, a broken row before seq_len raises."""
+    submission.clear_csr_cache()
+    B, H, T, lens = 2, 3, 1024, [700, 1024]
+    rp, ci = P.make_csr(B, H, T, lambda b, h, i: [] if i * 128 >= lens[b]
+                        else sorted({0, i // 2, i}))
+    q, k, v = P.make_qkv(B, H, T, seed=11)
+    dev = [x.cuda() for x in (q, k, v)] + [torch.from_numpy(x).cuda() for x in (rp, ci)]
+    sl = torch.tensor(lens, dtype=torch.int32, device="cpu" if on_host else "cuda")
+    calls = []
+    host = submission._check_on_host
+    monkeypatch.setattr(submission, "_check_on_host", lambda *a: (calls.append(1), host(*a)))
+    print(f"case rows end at seq_len, seq_lens on the host {on_host}", flush=True)
+    for _ in range(2):
+        o, l = block_sparse_attn_fwd(*dev, sl)
+        torch.cuda.synchronize()
+        oo, ol = c_ref.fwd(q.float().numpy(), k.float().numpy(), v.float().numpy(), rp, ci,
+                           np.asarray(lens, np.int32), round_p_fp16=False)
+        assert_close(o.float().cpu().numpy(), oo)
+        assert_close(l.cpu().numpy(), ol, what="LSE")
+    assert not calls and len(submission._csr_cache) == 1
+    with pytest.raises(ValueError, match="empty"):  # the same CSR does not do without seq_lens
+        block_sparse_attn_fwd(*dev, None)
+    with pytest.raises(ValueError, match="b=0,h=0,qb=6"):
+        block_sparse_attn_fwd(*dev, torch.tensor([800, 1024], dtype=torch.int32))
+    dev[4][1, 2, 5] = 7
+    with pytest.raises(ValueError, match="b=1,h=2"):
+        block_sparse_attn_fwd(*dev, sl)
+    submission.clear_csr_cache()

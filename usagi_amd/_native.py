@@ -24,6 +24,7 @@ EXPORTED_SYMBOLS = (
     "usagi_bsa_fwd_window",
     "usagi_bsa_check_csr",
     "usagi_bsa_check_csr_gpu",
+    "usagi_bsa_check_csr_gpu_lens",
     "usagi_bsa_plan",
     "usagi_bsa_time_next_launch",
     "usagi_bsa_version",
@@ -67,6 +68,8 @@ def load() -> ctypes.CDLL:
     lib.usagi_bsa_check_csr.restype = ctypes.c_int
     lib.usagi_bsa_check_csr_gpu.argtypes = [p, p, i32, i32, i32, i32, p, i32, p]
     lib.usagi_bsa_check_csr_gpu.restype = ctypes.c_int
+    lib.usagi_bsa_check_csr_gpu_lens.argtypes = [p, p, p, i32, i32, i32, i32, p, i32, p]
+    lib.usagi_bsa_check_csr_gpu_lens.restype = ctypes.c_int
     lib.usagi_bsa_plan.argtypes = [p, i32, i32, i32, i32, p, i32]
     lib.usagi_bsa_plan.restype = ctypes.c_int
     lib.usagi_bsa_time_next_launch.argtypes = [p, p]
@@ -153,6 +156,8 @@ def plan_host(row_ptr, batch: int, heads: int, nqb: int, generic: bool = False):
 
 # USAGI_BSA_CHECK_MAX_BLOCKS of include/usagi_bsa.h
 CHECK_MAX_BLOCKS = 8192
+# USAGI_BSA_CHECK_FLAG_BITS
+CHECK_FLAG_BITS = 4
 
 
 def check_cap(n_rows: int) -> int:
@@ -161,10 +166,11 @@ def check_cap(n_rows: int) -> int:
 
 
 def check_csr_gpu(row_ptr_ptr, col_idx_ptr, batch, heads, nqb, max_nnz, result_ptr, result_cap,
-                  stream) -> int:
-    """Launch the CSR check on the GPU; returns the number of flag words in the result."""
-    n = load().usagi_bsa_check_csr_gpu(row_ptr_ptr, col_idx_ptr, batch, heads, nqb, max_nnz,
-                                       result_ptr, result_cap, stream)
+                  stream, seq_lens_ptr=None) -> int:
+    """Launch the CSR check on the GPU (usagi_bsa_check_csr_gpu_lens); returns the number of flag words
+    in the result."""
+    n = load().usagi_bsa_check_csr_gpu_lens(row_ptr_ptr, col_idx_ptr, seq_lens_ptr, batch, heads, nqb,
+                                            max_nnz, result_ptr, result_cap, stream)
     if n <= 0:
         raise NativeError(n, last_error())
     return n

@@ -19,15 +19,20 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxBlocks = USAGI_BSA_CHECK_MAX_BLOCKS;
 constexpr int kMaxGroups = 1024;
+constexpr int kFlagBits = USAGI_BSA_CHECK_FLAG_BITS;
+constexpr int kMaxEntries = 0x7fffffff >> kFlagBits;  // above every row of kMaxBlocks full causal ones
 
 struct CheckArgs {
   const int32_t* row_ptr;
   const int32_t* col_idx;
+  const int32_t* seq_lens;  // or NULL: every row counts
   int32_t* result;
+  int heads;
   int bh_count;
   int nqb;
   int max_nnz;
   int groups;
+  int with_entries;  // the flag words hold the largest row end too
 };
 
 __global__ __launch_bounds__(kThreads) void bsa_check_kernel(CheckArgs a) {
@@ -63,19 +68,24 @@ __global__ __launch_bounds__(kThreads) void bsa_check_kernel(CheckArgs a) {
     }
   }
 
-  int bad = 0;
+  int bad = 0;   // 1: a row before seq_len, 4: one at or past it, which the walk never reads
   int differs = window == 0;
+  int entries = 0;  // largest end of a row
   for (int row = blockIdx.x * kWaves + wave; row < n_rows; row += a.groups * kWaves) {
     const int bh = row / nqb;
     const int qb = row - bh * nqb;
     const int32_t* rp = a.row_ptr + (size_t)bh * (nqb + 1) + qb;
     const int rs = rp[0];
     const int re = rp[1];
-    if (lane == 0) a.result[a.groups + 2 + row] = max(re - rs, 0);
-    if (!in_list(rs, re) || (qb == 0 && rs != 0)) {
-      bad = differs = 1;
+    const int bad_row = a.seq_lens && qb * USAGI_BSA_BLOCK >= a.seq_lens[bh / a.heads] ? 4 : 1;
+    const bool listless = !in_list(rs, re) || (qb == 0 && rs != 0);
+    if (lane == 0) a.result[a.groups + 2 + row] = listless && bad_row == 4 ? 0 : max(re - rs, 0);
+    if (listless) {
+      bad |= bad_row;
+      differs = 1;
       continue;
     }
+    entries = max(entries, re);
     const int n = re - rs;
     const int lo = max(qb - window + 1, 0);
     const int ng = min(n_global, lo);
@@ -96,15 +106,19 @@ __global__ __launch_bounds__(kThreads) void bsa_check_kernel(CheckArgs a) {
         wrong |= (atomicOr(&listed[wave][kb >> 5], 1u << (kb & 31)) >> (kb & 31)) & 1u;
       }
     }
-    if (wrong) bad = 1;
+    if (wrong) bad |= bad_row;
   }
-  const int f = (__any(bad) ? 1 : 0) | (__any(differs) ? 2 : 0);
-  if (lane == 0) flags[wave] = f;
+  const int f = (__any(bad & 1) ? 1 : 0) | (__any(differs) ? 2 : 0) | (__any(bad & 4) ? 4 : 0);
+  if (lane == 0) flags[wave] = min(entries, kMaxEntries) << kFlagBits | f;
   __syncthreads();
   if (threadIdx.x == 0) {
     int all = 0;
-    for (int w = 0; w < kWaves; ++w) all |= flags[w];
-    a.result[blockIdx.x] = all;
+    int most = 0;
+    for (int w = 0; w < kWaves; ++w) {
+      all |= flags[w] & ((1 << kFlagBits) - 1);
+      most = max(most, flags[w] >> kFlagBits);
+    }
+    a.result[blockIdx.x] = (a.with_entries ? most << kFlagBits : 0) | all;
     if (blockIdx.x == 0) {
       a.result[a.groups] = window;
       a.result[a.groups + 1] = n_global;
@@ -112,11 +126,9 @@ __global__ __launch_bounds__(kThreads) void bsa_check_kernel(CheckArgs a) {
   }
 }
 
-}  // namespace
-
-extern "C" int usagi_bsa_check_csr_gpu(const int32_t* row_ptr, const int32_t* col_idx, int32_t batch,
-                                       int32_t heads, int32_t num_q_blocks, int32_t max_nnz,
-                                       int32_t* result, int32_t result_cap, void* stream) {
+int launch_check(const int32_t* row_ptr, const int32_t* col_idx, const int32_t* seq_lens, int32_t batch,
+                 int32_t heads, int32_t num_q_blocks, int32_t max_nnz, int32_t* result,
+                 int32_t result_cap, void* stream, bool with_entries) {
   usagi_bsa_clear_error();
   if (!row_ptr || !result || batch <= 0 || heads <= 0 || num_q_blocks <= 0 || max_nnz < 0 ||
       (max_nnz > 0 && !col_idx))
@@ -128,6 +140,9 @@ extern "C" int usagi_bsa_check_csr_gpu(const int32_t* row_ptr, const int32_t* co
   CheckArgs a;
   a.row_ptr = row_ptr;
   a.col_idx = col_idx;
+  a.seq_lens = seq_lens;
+  a.heads = heads;
+  a.with_entries = with_entries ? 1 : 0;
   a.result = result;
   a.bh_count = (int)bh;
   a.nqb = num_q_blocks;
@@ -147,4 +162,21 @@ extern "C" int usagi_bsa_check_csr_gpu(const int32_t* row_ptr, const int32_t* co
     return -1000 - (int)err;
   }
   return a.groups;
+}
+
+}  // namespace
+
+extern "C" int usagi_bsa_check_csr_gpu(const int32_t* row_ptr, const int32_t* col_idx, int32_t batch,
+                                       int32_t heads, int32_t num_q_blocks, int32_t max_nnz,
+                                       int32_t* result, int32_t result_cap, void* stream) {
+  return launch_check(row_ptr, col_idx, nullptr, batch, heads, num_q_blocks, max_nnz, result, result_cap,
+                      stream, false);
+}
+
+extern "C" int usagi_bsa_check_csr_gpu_lens(const int32_t* row_ptr, const int32_t* col_idx,
+                                            const int32_t* seq_lens, int32_t batch, int32_t heads,
+                                            int32_t num_q_blocks, int32_t max_nnz, int32_t* result,
+                                            int32_t result_cap, void* stream) {
+  return launch_check(row_ptr, col_idx, seq_lens, batch, heads, num_q_blocks, max_nnz, result, result_cap,
+                      stream, true);
 }

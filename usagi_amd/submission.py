@@ -73,8 +73,6 @@ _raw_stream = torch._C._cuda_getCurrentRawStream
 
 _NOTHING = contextlib.nullcontext()
 
-_INT32_MAX = 2 ** 31 - 1
-
 # Query blocks up to which no work plan is made: they all run at once (one workgroup per CU or more).
 _PLAN_ITEMS = 256
 
@@ -110,6 +108,11 @@ class _CsrEntry:
         # The key of an entry that is not in the cache yet (else None): the call that made it checks
         # the CSR on the GPU (_start_check, _finish_check) around its launch.
         self.unchecked = None
+
+    def valid_before(self, seq_lens) -> None:
+        """Rows past seq_len may hold anything: the entry stands for calls with these seq_lens."""
+        self.seq_key, ref = _seq_key(seq_lens)
+        self.seq_ref = None if ref is None else weakref.ref(ref)
 
 
 _csr_cache: "OrderedDict[tuple, _CsrEntry]" = OrderedDict()
@@ -245,16 +248,16 @@ def _check_on_host(e: _CsrEntry, row_ptr, col_idx, B, H, nqb, dev, generic: bool
                 raise
             sl = torch.as_tensor(seq_lens).detach().to("cpu", torch.int32).reshape(-1).numpy()
             _native.check_csr_host(rp, ci, B, H, nqb, max_nnz, seq_lens=sl)
-            e.seq_key, sref = _seq_key(seq_lens)
-            e.seq_ref = None if sref is None else weakref.ref(sref)
+            e.valid_before(seq_lens)
     _plan_entry(e, rp, ci, B, H, nqb, dev, generic)
 
 
-def _start_check(result, rp, ci, B, H, nqb, max_nnz, stream) -> tuple:
+def _start_check(result, rp, ci, sl, B, H, nqb, max_nnz, stream) -> tuple:
     """Launch the GPU check of int32 device tensors; the forward launch follows it on the stream.
     result: pinned memory that the caller keeps until the check has run."""
     n_flags = _native.check_csr_gpu(rp.data_ptr(), ci.data_ptr(), B, H, nqb, max_nnz,
-                                    result.data_ptr(), result.numel(), stream)
+                                    result.data_ptr(), result.numel(), stream,
+                                    sl.data_ptr() if sl is not None else None)
     done = torch.cuda.Event()
     done.record()
     return done, result, n_flags
@@ -264,7 +267,7 @@ def _finish_check(e: _CsrEntry, check: tuple, row_ptr, col_idx, B, H, nqb, dev, 
                   seq_lens) -> None:
     """Wait for the check (the forward kernel is queued behind it or running), keep what it found in
     the entry and the entry in the cache; a CSR that it rejects is looked at again on the host, which
-    raises with the row's position or accepts the rows before seq_len."""
+    raises with the row's position."""
     import numpy as np
 
     done, result, n_flags = check
@@ -275,12 +278,13 @@ def _finish_check(e: _CsrEntry, check: tuple, row_ptr, col_idx, B, H, nqb, dev, 
     if flags & 1 and not generic:
         _check_on_host(e, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
     else:
+        if flags & 4 and not generic:
+            e.valid_before(seq_lens)
         rows = B * H * nqb
-        lengths = r[n_flags + 2:n_flags + 2 + rows].reshape(B * H, nqb)
-        e.entries = min(int(lengths.sum(axis=1, dtype=np.int64).max()), _INT32_MAX)
+        e.entries = int(r[:n_flags].max()) >> _native.CHECK_FLAG_BITS
         if rows > _PLAN_ITEMS:
             rp = np.zeros((B * H, nqb + 1), dtype=np.int32)
-            np.cumsum(lengths, axis=1, out=rp[:, 1:])
+            np.cumsum(r[n_flags + 2:n_flags + 2 + rows].reshape(B * H, nqb), axis=1, out=rp[:, 1:])
             _plan_rows(e, rp, B, H, nqb, dev, generic, pinned=True)
         if not generic and ROUTE_WINDOW and not flags & 2 and e.sched is None:
             e.window = (int(r[n_flags]), int(r[n_flags + 1]))
@@ -428,7 +432,7 @@ def _run_csr(q, k, v, row_ptr, col_idx, seq_lens, generic: bool):
             return out, lse
         result = torch.empty(_native.check_cap(B * H * nqb), dtype=torch.int32, pin_memory=True)
         try:
-            check = _start_check(result, rp, ci, B, H, nqb, max_nnz, stream)
+            check = _start_check(result, rp, ci, sl, B, H, nqb, max_nnz, stream)
             launch(-1)
             _finish_check(plan, check, row_ptr, col_idx, B, H, nqb, dev, generic, seq_lens)
         except BaseException:
