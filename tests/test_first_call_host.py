@@ -4,6 +4,9 @@ whatever raises before the result is read. The device calls are stand-ins that n
 from __future__ import annotations
 
 import contextlib
+import os
+import subprocess
+import sys
 import weakref
 
 import pytest
@@ -11,6 +14,8 @@ import torch
 
 from usagi_amd import _native, submission
 from usagi_amd import patterns as P
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 class FakeGpu:
@@ -76,3 +81,16 @@ def test_a_queued_check_outlives_no_error(monkeypatch, fail, error):
     del caught
     assert gpu.released_while == [False] and not gpu.queued
     assert not submission._csr_cache  # nothing is kept of a CSR that was not checked
+
+
+def test_import_needs_no_private_torch_name():
+    """A torch without its ROCm parts lacks _cuda_getCurrentRawStream; the planner, the patterns and the
+    host check are there all the same."""
+    code = ("import torch\n"
+            "del torch._C._cuda_getCurrentRawStream\n"
+            "import usagi_amd\n"
+            "from usagi_amd import _native, patterns as P\n"
+            "rp, ci = P.sliding_csr(1, 2, 512, 2)\n"
+            "_native.check_csr_host(rp, ci, 1, 2, 4, ci.shape[-1])\n")
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=REPO)
+    assert res.returncode == 0, res.stderr[-2000:]

@@ -68,8 +68,10 @@ _DTYPE_CODES = {torch.float16: _native.FP16, torch.bfloat16: _native.BF16}
 
 _CSR_CACHE_SIZE = 64
 
-# Handle of the current stream of a device (by index), as torch.cuda.current_stream().cuda_stream.
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# Handle of the current stream of a device (by index), as torch.cuda.current_stream().cuda_stream; torch's
+# own short cut to it (no Stream object: 0.05 us a call instead of 2.1) where it is there.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                      lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 _NOTHING = contextlib.nullcontext()
 
