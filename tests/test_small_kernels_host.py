@@ -78,3 +78,11 @@ def test_kernel_of_and_fwd_entries_reject_what_the_forward_rejects():
         assert lib.usagi_bsa_kernel_of(B, H, T, 0, nnz, 0, -1) < 0 and _native.last_error()
         assert lib.usagi_bsa_fwd_entries(1, 1, 1, 1, 1, None, 1, None, B, H, T, 128, nnz, 0, None, 0, None,
                                          0, 1) < 0
+
+
+def test_generic_rows_of_one_block_take_the_small_kernels_up_to_64_query_blocks():
+    for H, nqb, want in ((4, 8, 32), (8, 8, 32), (9, 8, 0), (16, 8, 0)):
+        T = nqb * 128
+        assert _native.kernel_of(1, H, T, False, nqb, True) == want
+        assert _native.kernel_of(1, H, T, False, 2 * nqb, True) == (want or 64)
+        assert _native.kernel_of(1, H, T, True, nqb, False) == (want or 64)

@@ -924,8 +924,17 @@ LaunchEvents take_events() {
 //   n = 128, T 4096, w 16: dma 32.2 / 40.2                  32: 26.2 / 30.3  64: 21.0 / 24.6
 //   n = 256, T 4096, w 16: dma 32.4 / 40.1                  64: 40.8 / 48.7  128: 30.5 / 32.5
 //   n = 256, T 1024, w 4:  dma 12.6 / 14.4                                   128: 13.1 / 14.5
-// so the line to 32 rows lies at 64 query blocks (256 workgroups, one per CU), to 64 rows at 128
-// and to 128 rows at 256, the last only for rows of 6 blocks and more. Long rows that grow towards the
+// short rows with seq_lens (no pipelined kernel) and on the generic walk (T 1024):
+//   n = 32,  w 1:          dma  7.6 /  7.9                  32: 5.4 / 5.5
+//   n = 64,  w 2:          dma  9.6 / 10.3                  32: 7.2 / 7.4
+//   n = 72,  w 1:          dma  7.7 /  8.2                                   64: 7.3 / 7.7
+//   n = 128, w 1:          dma  7.8 /  8.2                                   64: 7.6 / 8.0
+//   n = 128, w 2:          dma 10.0 / 10.5                                   64: 9.4 / 9.7
+//   n = 128, w 1, generic: dma  7.3 /  7.8                                   64: 7.8 / 8.0
+//   n = 128, w 2, generic: dma  9.4 / 10.1                                   64: 9.4 / 9.8
+// so the line to 32 rows lies at 64 query blocks (256 workgroups, one per CU), to 64 rows at 128 (not
+// for generic rows of one block, where there is no chain to shorten and the merge is extra) and to 128
+// rows at 256, the last only for rows of 6 blocks and more. Long rows that grow towards the
 // end of the sequence leave the chip emptier still: full causal rows of 32 blocks take 36 (64 rows)
 // against 52 (128) at n = 160 and 44 against 52 at n = 256 (of 8 blocks at n = 256: 24 against 18), and
 // where two workgroups of bsa_fwd_dma_kernel share a CU until the longest row ends (n = 512: 89 / 102
@@ -958,9 +967,9 @@ double causal_row(long long entries, int nqb) {
 // Query rows per workgroup of the bsa_ksplit.hip kernel for this call, 0: none of them.
 int small_query_rows(const Args& a, int kRows, long long entries) {
   if (a.n_items <= kSmall32) return 32;
-  if (a.n_items <= kSmall64) return 64;
-  if (a.n_items > kSmallCausal) return 0;
   const double mean = (double)entries / a.nqb;
+  if (a.n_items <= kSmall64) return kRows == kRowsGeneric && mean < 1.5 ? 0 : 64;
+  if (a.n_items > kSmallCausal) return 0;
   const double longest = kRows == kRowsGeneric ? mean : causal_row(entries, a.nqb);
   if (a.n_items <= kSmall128) {
     if (longest < 6.0) return 0;
