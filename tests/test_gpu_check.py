@@ -1,6 +1,7 @@
 """The CSR check on the GPU against the host check, window_pattern and the CSR itself: valid rows,
 rows broken in each way the host check names, window and near-window patterns, rows longer than a
-wave, few and many rows per wave; and the first call of the shim around it."""
+wave, few and many rows per wave, rows past seq_len; the first call of the shim around it (padded lists,
+rows that end at seq_len) and captured calls after it."""
 
 from __future__ import annotations
 
@@ -237,4 +238,40 @@ def test_rows_that_end_at_seq_len_are_checked_on_the_gpu(on_host, monkeypatch):
     dev[4][1, 2, 5] = 7
     with pytest.raises(ValueError, match="b=1,h=2"):
         block_sparse_attn_fwd(*dev, sl)
+    submission.clear_csr_cache()
+
+
+@pytest.mark.parametrize("case", ["plan", "few query blocks", "padded", "rows end at seq_len"])
+def test_calls_captured_after_a_first_call(case):
+    """A CSR seen before is launched from its cache entry under stream capture; every replay, with eager
+    work between them, gives the eager result."""
+    submission.clear_csr_cache()
+    sl = None
+    if case == "plan":
+        rp, ci = P.mixed_csr(1, 16, 4096, 3)
+    elif case == "few query blocks":
+        rp, ci = P.retrieval_csr(1, 4, 2048, 6, 1)
+    elif case == "padded":
+        rp, ci = P.retrieval_csr(1, 8, 4096, 6, 1)
+        ci = np.concatenate([ci, np.zeros((1, 8, 400), np.int32)], axis=-1)
+    else:
+        rp, ci = P.make_csr(2, 3, 1024, lambda b, h, i: [] if i * 128 >= 700 else sorted({0, i // 2, i}))
+        sl = torch.tensor([700, 650], dtype=torch.int32, device="cuda")
+    B, H, n1 = rp.shape
+    dev = [x.cuda() for x in P.make_qkv(B, H, (n1 - 1) * 128, seed=2)]
+    dev += [torch.from_numpy(x).cuda() for x in (rp, ci)] + [sl]
+    print(f"case captured {case}", flush=True)
+    want, want_lse = block_sparse_attn_fwd(*dev)
+    torch.cuda.synchronize()
+    assert (next(iter(submission._csr_cache.values())).sched is not None) == (case == "plan")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        o, lse = block_sparse_attn_fwd(*dev)
+    for _ in range(4):
+        o.zero_()
+        lse.zero_()
+        block_sparse_attn_fwd(*dev)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want) and torch.equal(lse, want_lse)
     submission.clear_csr_cache()

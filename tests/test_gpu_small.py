@@ -1,7 +1,7 @@
 """The kernels for few query blocks (bsa_ksplit.hip) at the sizes where their choice or their tiling
 changes: 64 / 128 / 256 / 512 query blocks, counts that are no multiple of 8, rows of 1, 2, 3 and more
 than 64 blocks, rows without their diagonal, and sequences cut inside and between the 32- and 64-row
-parts of a query block. Against the fp32 walk; atol = rtol = 2e-3, half a bf16 ulp more for bf16 O."""
+parts of a query block, NaN and infinities past seq_len. Against the fp32 walk; atol = rtol = 2e-3, half a bf16 ulp more for bf16 O."""
 
 from __future__ import annotations
 

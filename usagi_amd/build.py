@@ -44,8 +44,10 @@ def hipcc_command(srcs: list[str] | None = None, out: str = LIB_PATH,
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         # MFMA accumulators stay in VGPRs while they fit, instead of being copied out of AGPRs.
         "-mllvm", "-amdgpu-mfma-vgpr-form",
-        # The key loop of bsa_fwd_dma_kernel is instruction-fetch sensitive: started on a 64-byte line,
-        # rows of 80 bf16 blocks take 287 us instead of 305, retrieval rows 230 instead of 233.
+        # The key loop of bsa_fwd_dma_kernel is instruction-fetch sensitive: where code ahead of it had
+        # moved its start off a 64-byte line, rows of 80 bf16 blocks took 305 us instead of 287. With the
+        # code as it is now the flag changes nothing there (288.2 us without it, 287.6 with), and bf16
+        # retrieval rows with seq_lens take 191 instead of 193: it keeps later changes from moving it.
         "-falign-loops=64",
         "-I", INCLUDE_DIR,
         "-I", CSRC_DIR,

@@ -134,7 +134,6 @@ __device__ __forceinline__ floatx4 mfma_qk16(u32x4 a, u32x4 b, floatx4 c) {
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
 typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_cvoid;
 
 // One 16-byte-per-lane DMA: global (uniform base + per-lane byte offset) -> LDS at the uniform
 // byte address lds_addr + 16 * lane. Issued as inline asm so that the compiler's wait-count pass
@@ -188,7 +187,6 @@ __device__ __forceinline__ void zero_v_tail(char* slice, int lane, int from) {
 
 #define USAGI_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 #define USAGI_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
-#define USAGI_FENCE() __builtin_amdgcn_sched_barrier(0)
 
 // Rows of one query block (kRows):
 //   kRowsCsr     the CSR walk of kernels/v7_blockptr_warpspec.py:77-136: entries before the last

@@ -93,7 +93,9 @@ void bsa_fwd_dma_kernel(Args a) {
   // saves the DMA's LDS write and the conversion's LDS read, or in place after its DMA. Through
   // registers is 1-3% faster on analytic rows (sliding w8 B2 H16 T8192: 142.5 against 145.0 us) and
   // generic rows (128.4 against 131.6), but not on CSR rows (rows of 80 blocks, B1 H2 T32768: 290
-  // against 286), whose column registers leave the scheduler less room.
+  // against 286), whose column registers leave the scheduler less room. Other CSR rows go both ways:
+  // retrieval B2 H16 T8192 230.6 against 231.9 (with seq_lens 188.8 against 191.6), rows of 8 B4 H16 T2048
+  // with seq_lens 54.7 against 53.4.
   constexpr bool kVRegs = kBf16 && kRows != kRowsCsr;
 
   const int tid = threadIdx.x;

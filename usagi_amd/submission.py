@@ -75,7 +75,10 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
 
 _NOTHING = contextlib.nullcontext()
 
-# Query blocks up to which no work plan is made: they all run at once (one workgroup per CU or more).
+# Query blocks up to which no work plan is made. All workgroups then run at once, but for the kernel with two
+# per query block at 129 .. 256 query blocks (long growing rows), whose second half waits for a CU: there a
+# plan can help (one full causal head of 8, T 4096: 35 us against 46) or hurt as much (two full causal heads,
+# T 16384: 239 against 157), and mostly does neither (heads of mixed patterns, T 4096: 45.7 against 45.6).
 _PLAN_ITEMS = 256
 
 
