@@ -11,7 +11,8 @@ import torch
 
 from tests._helpers import assert_close
 from oracle import c_ref
-from usagi_amd import _native, block_sparse_attn_fwd, submission
+from usagi_amd import (_native, block_sparse_attn_fwd, block_sparse_attn_fwd_generic,
+                       submission)
 from usagi_amd import patterns as P
 
 pytestmark = pytest.mark.gpu
@@ -275,3 +276,14 @@ def test_calls_captured_after_a_first_call(case):
         torch.cuda.synchronize()
         assert torch.equal(o, want) and torch.equal(lse, want_lse)
     submission.clear_csr_cache()
+
+
+@pytest.mark.parametrize("on_host", [False, True])
+def test_an_empty_batch_is_rejected_as_before_the_gpu_check(on_host):
+    q = torch.empty((0, 3, 1024, 128), dtype=torch.float16, device="cuda")
+    dev = "cpu" if on_host else "cuda"
+    rp, ci = (torch.empty((0, 3, n), dtype=torch.int32, device=dev) for n in (9, 20))
+    with pytest.raises(ValueError):
+        block_sparse_attn_fwd(q, q, q, rp, ci, None)
+    with pytest.raises(_native.NativeError):
+        block_sparse_attn_fwd_generic(q, q, q, rp, ci, None)

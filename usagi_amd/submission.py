@@ -232,9 +232,10 @@ def _remember(e: _CsrEntry, key: tuple) -> None:
 
 
 def _on_gpu(row_ptr, col_idx, dev, nqb: int, max_nnz: int) -> bool:
-    """Whether the CSR can be checked on the GPU: there already, and not under stream capture (the
-    result is waited for)."""
-    return (dev.type == "cuda" and row_ptr.device == dev and col_idx.device == dev and max_nnz > 0
+    """Whether the CSR can be checked on the GPU: there already, with any rows, and not under stream
+    capture (the result is waited for)."""
+    return (dev.type == "cuda" and row_ptr.device == dev and col_idx.device == dev
+            and max_nnz > 0 and row_ptr.numel() > 0
             and nqb <= _native.CHECK_MAX_BLOCKS and not torch.cuda.is_current_stream_capturing())
 
 
@@ -317,7 +318,7 @@ def _plan_rows(e: _CsrEntry, rp, B, H, nqb, dev, generic: bool, pinned=False) ->
 
 def _plan_entry(e: _CsrEntry, rp, ci, B, H, nqb, dev, generic: bool, pinned=False) -> None:
     """Entries, work plan and window pattern of a host copy of the CSR, into the entry."""
-    e.entries = max(int(rp.max()), 0)
+    e.entries = max(int(rp.max(initial=0)), 0)
     _plan_rows(e, rp, B, H, nqb, dev, generic, pinned)
     if e.sched is None and not generic and ROUTE_WINDOW and ci.shape[-1]:
         e.window = window_pattern(rp, ci, nqb)
